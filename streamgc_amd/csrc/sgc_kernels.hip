@@ -517,20 +517,185 @@ __global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ 
     if (grouped && totals && lane() == 0) tot_add(totals, T_GROUPED, grouped);
 }
 
-// One wavefront per segment, the segment's updates in order; positions go
-// through `perm` when given (per-graph order inside a mixed batch).
-__global__ __launch_bounds__(256) void k_apply_seg(const GraphDev* __restrict__ graphs,
-                                                   const uint4* __restrict__ upd, const uint32_t* __restrict__ seg,
-                                                   uint32_t nseg, const uint32_t* __restrict__ perm, int multi,
-                                                   uint64_t* totals, const uint32_t* __restrict__ dyn) {
+__device__ __forceinline__ uint4 uniform_rec(const uint4& r) {
+    return make_uint4(bcast0(r.x), bcast0(r.y), bcast0(r.z), bcast0(r.w));
+}
+
+// One block per segment, the segment's updates in stream order (deterministic
+// mode); positions go through `perm` when given (per-graph order inside a
+// mixed batch).  One wavefront replaying a segment spends its time on one
+// update's chain of dependent loads at a time (2.6 us an update, whatever the
+// graph's size), so the block's WAVES wavefronts take the next WAVES updates
+// and judge each at once, reading only (replay_plain): an update is plain if it
+// changes no word and finds room in both rows, whatever the plain updates
+// before it in the window do.  Plain updates touch nothing but their own
+// endpoints' rows, fills, bitmaps, histograms and marks, so those before the
+// first that is not plain run a wavefront each, in rounds: an update waits only
+// for the earlier ones that share an endpoint with it.  The first that is not
+// plain then runs alone.  The result is the one-at-a-time replay's, slot for
+// slot.  After a window whose first update was not plain (a stream that colours
+// fresh vertices), wavefront 0 applies the next updates alone, twice as many
+// after each such window up to REPLAY_ALONE, so that a stream with nothing to
+// run together pays for few judgements.  Measured against one wavefront a
+// segment: 509 updates of a 16,384-vertex mesh with their epoch step 1,420 ->
+// 425 us; 48 graphs of 2^10..2^14 vertices, 71K updates, 11.1 -> 4.7 ms.
+constexpr uint32_t REPLAY_WAVES = 16;    // 4 wavefronts per SIMD, what one update's registers allow
+constexpr uint32_t REPLAY_CHUNK = 256;   // records staged in LDS at a time
+constexpr uint32_t REPLAY_ALONE = 64;
+
+template <uint32_t WAVES>
+struct ReplayWindow {
+    uint4 recs[REPLAY_CHUNK];
+    // of each update of the window: its endpoints (INVALID: it changes nothing)
+    // and their colours, whether it is an insert, the earlier ones it shares an
+    // endpoint with, whether it is plain
+    uint32_t end[2 * WAVES], col[2 * WAVES], ins[WAVES], after[WAVES], plain[WAVES];
+};
+
+// Whether the removal of a neighbour coloured `freed` leaves vertex x (colour
+// cur) its colour, after the window's earlier updates of x (a lane each: they
+// take or give a neighbour coloured `other`; `mine` says which lanes).
+// Bitmap mode: no bit below cur is clear (bits are only ever added) and a bit
+// stays clear whatever the earlier inserts add.  Histogram mode: no bin below
+// cur's that is or becomes zero.
+__device__ __forceinline__ bool keeps_colour(const GraphDev& g, uint32_t hd, uint64_t bits, uint16_t freed,
+                                             uint16_t cur, uint64_t mine, uint64_t inserts, uint32_t other) {
+    if (cur == 0 || freed >= cur) return true;   // try_reduce does nothing
+    if (hd == INVALID || (g.flags & ABL_FORCE_BITMAP))
+        return (uint32_t)__builtin_popcountll(~bits) > (uint32_t)__builtin_popcountll(inserts) &&
+               (uint32_t)__builtin_ctzll(~bits) + 1u >= cur;
+    if (cur > HIST_BINS) return false;
+    const uint32_t* h = g.hist + (size_t)hd * HIST_BINS;
+    for (uint32_t k = 0; k + 1 < cur; k += WAVE) {
+        const uint32_t c = k + lane() + 1;
+        uint32_t left = c < cur ? ld(&h[c - 1]) - (c == freed ? 1u : 0u) : 1u;
+        for (uint64_t m = mine; m; m &= m - 1) {
+            const uint32_t i = (uint32_t)__builtin_ctzll(m);
+            const uint32_t at = __builtin_amdgcn_readlane(other, i);
+            if (c < cur && at == c) left += (inserts >> i) & 1 ? 1u : 0xFFFFFFFFu;
+        }
+        if (ballot(left == 0)) return false;
+    }
+    return true;
+}
+
+// Judge the window's update of wavefront wv (every wavefront of the block calls it).
+template <uint32_t WAVES>
+__device__ __forceinline__ void replay_judge(const GraphDev& g, const uint4& r, bool have, uint32_t wv,
+                                             ReplayWindow<WAVES>& w) {
+    const uint32_t u = r.x, v = r.y, type = r.z & 0xFFu;
+    const bool none = !have || u >= g.n || v >= g.n || type > 1;   // touches no vertex
+    uint32_t room_u = 0, room_v = 0, hu = INVALID, hv = INVALID, wu = 0, wv0 = 0, fu = 0, fv = 0;
+    uint64_t bu = 0, bv = 0;
+    if (!none) {
+        room_u = gp(g.row_ptr)[u + 1] - gp(g.row_ptr)[u], room_v = gp(g.row_ptr)[v + 1] - gp(g.row_ptr)[v];
+        hu = gp(g.hd_map)[u], hv = gp(g.hd_map)[v];
+        wu = ld(&g.word[u]), wv0 = ld(&g.word[v]);
+        fu = ld(&g.fill[u]), fv = ld(&g.fill[v]);
+        bu = ld(&g.bitmap[u]), bv = ld(&g.bitmap[v]);
+    }
+    const uint16_t cu = color_of(bcast0(wu)), cv = color_of(bcast0(wv0));
+    if (lane() == 0) {
+        w.end[2 * wv] = none ? INVALID : u;
+        w.end[2 * wv + 1] = none ? INVALID : v;
+        w.col[2 * wv] = cu;
+        w.col[2 * wv + 1] = cv;
+        w.ins[wv] = type == 0;
+    }
+    __syncthreads();
+    // lane i: the window's update i, if it comes before this one
+    const bool before = lane() < wv && !none;
+    const uint32_t i = before ? lane() : 0;
+    const uint32_t iu = w.end[2 * i], iv = w.end[2 * i + 1];
+    const bool at_u = before && iu != INVALID && (iu == u || iv == u);
+    const bool at_v = before && iu != INVALID && (iu == v || iv == v);
+    const uint64_t mu = ballot(at_u), mv = ballot(at_v), mi = ballot(before && w.ins[i] != 0);
+    bool ok = have;
+    if (!none) {
+        if (u == v) {
+            ok = false;
+        } else if (type == 0) {
+            ok = cu != 0 && cv != 0 && cu != cv && bcast0(fu) + (uint32_t)__builtin_popcountll(mu & mi) < bcast0(room_u) &&
+                 bcast0(fv) + (uint32_t)__builtin_popcountll(mv & mi) < bcast0(room_v);
+        } else {
+            const uint32_t ou = iu == u ? w.col[2 * i + 1] : w.col[2 * i];   // the other endpoint's colour
+            const uint32_t ov = iu == v ? w.col[2 * i + 1] : w.col[2 * i];
+            ok = keeps_colour(g, hu, bu, cv, cu, mu, mu & mi, ou) && keeps_colour(g, hv, bv, cu, cv, mv, mv & mi, ov);
+        }
+    }
+    if (lane() == 0) {
+        w.after[wv] = (uint32_t)(mu | mv);
+        w.plain[wv] = ok ? 1u : 0u;
+    }
+    __syncthreads();
+}
+
+template <uint32_t WAVES>
+__global__ __launch_bounds__(WAVES * WAVE) void k_apply_seg(const GraphDev* __restrict__ graphs,
+                                                           const uint4* __restrict__ upd,
+                                                           const uint32_t* __restrict__ seg, uint32_t nseg,
+                                                           const uint32_t* __restrict__ perm, int multi,
+                                                           uint64_t* totals, const uint32_t* __restrict__ dyn) {
+    __shared__ ReplayWindow<WAVES> w;
     WaveAcc acc;
     if (dyn) {   // segments of the current round (absolute stream positions); none when its count is 0
         if (dyn[1] == 0) return;
         seg += dyn[2];
     }
-    for (uint32_t k = wave_id(); k < nseg; k += wave_count())
-        for (uint32_t i = seg[2 * k]; i < seg[2 * k + 1]; i++)
-            apply_record(graphs, upd, perm ? perm[i] : i, multi, acc);
+    const uint32_t wv = bcast0(threadIdx.x / WAVE);
+    for (uint32_t k = blockIdx.x; k < nseg; k += gridDim.x) {
+        uint32_t alone = 0, backoff = 1;
+        const uint32_t first = seg[2 * k], last = seg[2 * k + 1];
+        for (uint32_t base = first; base < last; base += REPLAY_CHUNK) {
+            const uint32_t cnt = last - base < REPLAY_CHUNK ? last - base : REPLAY_CHUNK;
+            __syncthreads();   // the chunk before is done with
+            for (uint32_t t = threadIdx.x; t < cnt; t += WAVES * WAVE)
+                w.recs[t] = upd[perm ? perm[base + t] : base + t];
+            __syncthreads();
+            for (uint32_t i0 = 0; i0 < cnt;) {   // (block-uniform)
+                uint32_t stop = 0, run = 1;      // `stop` updates in rounds, then `run` one after the other
+                if (WAVES == 1) {
+                    run = cnt - i0;
+                } else if (alone) {
+                    run = alone < cnt - i0 ? alone : cnt - i0;
+                    alone -= run;
+                } else if (cnt - i0 > 1) {
+                    const bool have = i0 + wv < cnt;
+                    const uint4 r = uniform_rec(w.recs[have ? i0 + wv : i0]);
+                    replay_judge(graphs[multi ? r.w : 0u], r, have, wv, w);
+                    stop = (uint32_t)__builtin_ctzll(~ballot(lane() < WAVES && w.plain[lane() < WAVES ? lane() : 0]));
+                    if (stop == WAVES || i0 + stop == cnt) run = 0;
+                    if (stop) {
+                        backoff = 1;
+                    } else {
+                        alone = backoff;
+                        backoff = backoff < REPLAY_ALONE ? 2 * backoff : REPLAY_ALONE;
+                    }
+                }
+                // One call site for all: a second copy of the update's code
+                // would not stay in the instruction cache beside the first.
+                const uint32_t wait = lane() < stop ? w.after[lane()] : 0u;
+                uint32_t done = 0;
+                const uint32_t all = (1u << stop) - 1u;
+                while (done != all || run) {
+                    uint32_t at = i0 + wv, mine;
+                    if (done != all) {
+                        const uint32_t ready = (uint32_t)ballot(lane() < stop && (wait & ~done) == 0) & ~done;
+                        mine = (ready >> wv) & 1u;
+                        done |= ready;
+                    } else {
+                        at = i0 + stop;
+                        mine = wv == 0 ? run : 0u;
+                        i0 += run;
+                        run = 0;
+                    }
+                    for (uint32_t i = at; i < at + mine; i++) apply_rec(graphs, uniform_rec(w.recs[i]), multi, acc);
+                    __syncthreads();
+                }
+                i0 += stop;
+            }
+        }
+    }
     acc.flush(totals);
 }
 
@@ -1875,11 +2040,22 @@ hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int
                                                eg->nheads, eg->pack, L.dyn);
     return hipGetLastError();
 }
+// Up to so many segments a block of wavefronts replays each, above it one
+// wavefront: with more segments than that the chip's wavefront slots are better
+// filled by one a segment (64 churn updates on each of n 200-vertex meshes, us
+// by blocks / by single wavefronts: 256: 50 / 155, 1024: 188 / 190, 2048:
+// 372 / 230; a stream that colours fresh vertices breaks even near 500).
+constexpr uint32_t REPLAY_MANY = 512;
 hipError_t launch_apply_seg(const LaunchCtx& L, const void* upd, const uint32_t* seg, uint32_t nseg,
                             const uint32_t* perm, int multi) {
     if (nseg == 0) return hipSuccess;
-    uint32_t grid = grid_for_waves(nseg, 1, L.max_blocks);
-    k_apply_seg<<<grid, 64, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg, perm, multi, L.totals, L.dyn);
+    const uint32_t grid = grid_for_waves(nseg, 1, L.max_blocks);
+    if (nseg <= REPLAY_MANY)
+        k_apply_seg<REPLAY_WAVES><<<grid, REPLAY_WAVES * WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg,
+                                                                              perm, multi, L.totals, L.dyn);
+    else
+        k_apply_seg<1><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg, perm, multi, L.totals,
+                                                    L.dyn);
     return hipGetLastError();
 }
 hipError_t launch_zero_ctr(const LaunchCtx& L, uint32_t idx) {
