@@ -65,6 +65,45 @@ __device__ __forceinline__ uint32_t sweep_big(const SweepList& sl) { return sl.l
 __device__ __forceinline__ uint32_t small_item(const SweepList& sl, uint32_t k) { return sl.list ? sl.list[k] : k; }
 __device__ __forceinline__ uint32_t big_item(const SweepList& sl, uint32_t k) { return sl.list[sl.cap - 1 - k]; }
 
+// The front rows of a sweep set (or every row) over the grid's wavefronts.
+// Rows are short -- 6 slots on a mesh, 17 on a social graph -- and a row is one
+// chain of dependent loads (list entry, row bounds, slots, neighbours' words),
+// so a wavefront takes four rows at a time, 16 lanes each; a grid with more
+// wavefronts than rows takes one each.  A full sweep of 4.0M rows and 69M live
+// slots, one row a wavefront / four: compaction 1,180 / 324 us, rebuild 2,200 /
+// 1,137 us, Tier-1 3,513 / 1,071 us (what is left is the gather of 69M
+// neighbour words).  body(g, gid, mine, v) runs with g wave-uniform (rows of several graphs: one graph after another): mine says
+// whether the lane's row v takes part.
+constexpr uint32_t GROUP = 16, GROUPS = WAVE / GROUP;
+constexpr uint32_t GROUP_ROW = ROW_UNROLL * GROUP;   // slots 16 lanes load in one round trip
+__device__ __forceinline__ uint32_t sublane() { return lane() % GROUP; }
+__device__ __forceinline__ uint32_t group_bits(uint64_t m) {   // the lane's group's bits of a ballot
+    return (uint32_t)(m >> (lane() / GROUP * GROUP)) & 0xFFFFu;
+}
+template <class F>
+__device__ __forceinline__ void for_rows(const GraphDev* __restrict__ graphs, const Space& sp, const SweepList& sl,
+                                         F&& body) {
+    const uint32_t total = sweep_small(sl, sp.total);
+    const uint32_t per = total > wave_count() ? GROUPS : 1u, mine_of = lane() / GROUP;
+    for (uint32_t k0 = wave_id() * per; k0 < total; k0 += wave_count() * per) {
+        const bool have = mine_of < per && k0 + mine_of < total;
+        uint32_t gid = 0, v = 0;
+        if (have) sp.locate(small_item(sl, k0 + mine_of), gid, v);
+        uint64_t pend = ballot(have);
+        while (pend) {
+            const uint32_t g0 = __builtin_amdgcn_readlane(gid, (uint32_t)__builtin_ctzll(pend));
+            const bool mine = have && gid == g0;
+            pend &= ~ballot(mine);
+            body(graphs[g0], g0, mine, v);
+        }
+    }
+}
+// The rows of `m` (a lane mask), one after another by the whole wavefront: f(v).
+template <class F>
+__device__ __forceinline__ void each_row(uint64_t m, uint32_t v, F&& f) {
+    for (; m; m &= m - 1) f((uint32_t)__builtin_amdgcn_readlane(v, (uint32_t)__builtin_ctzll(m)));
+}
+
 // Block-wide sum of per-wave values into one u64 total (one atomic per block).
 // Every thread of the block must call it.
 __device__ __forceinline__ void block_add64(uint64_t* totals, uint32_t idx, uint64_t mine) {
@@ -890,6 +929,31 @@ __device__ __forceinline__ uint32_t compact_row_wave(const GraphDev& g, uint32_t
     return w - s;
 }
 
+// Rows of at most GROUP_ROW slots, 16 lanes each: the lane's row of vertex v,
+// if `mine` (slots [s, s + f)).  Returns the row's live count.
+__device__ __forceinline__ uint32_t compact_row_group(const GraphDev& g, bool mine, uint32_t v, uint32_t s, uint32_t f) {
+    uint32_t val[ROW_UNROLL];
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t j = u * GROUP + sublane();
+        val[u] = mine && j < f ? gp(g.col)[s + j] : INVALID;
+    }
+    uint32_t w = s;
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t j = s + u * GROUP + sublane();
+        const bool live = val[u] != INVALID;
+        const uint32_t m = group_bits(ballot(live));
+        const uint32_t pos = w + (uint32_t)__builtin_popcount(m & ((1u << sublane()) - 1u));
+        const uint32_t w_after = w + (uint32_t)__builtin_popcount(m);
+        if (live && pos != j) gp(g.col)[pos] = val[u];
+        if (live && pos != j && j >= w_after) gp(g.col)[j] = INVALID;
+        w = w_after;
+    }
+    if (mine && sublane() == 0) gp(g.fill)[v] = w - s;
+    return w - s;
+}
+
 // The drain's counter snapshot of one graph (A/src/streamgc.cu:972-983): the
 // overflow entries it retries (capped at the buffer), those lost past the
 // buffer, counters reset.
@@ -926,16 +990,22 @@ __global__ __launch_bounds__(256) void k_compact(const GraphDev* __restrict__ gr
             slots += f;
         }
     }
-    const uint32_t total = sweep_small(sl, sp.total);
-    for (uint32_t k = wave_id(); k < total; k += wave_count()) {
-        uint32_t gid, v;
-        sp.locate(small_item(sl, k), gid, v);
-        const GraphDev& g = graphs[gid];
-        const uint32_t f = gp(g.fill)[v];
-        live_total += compact_row_wave(g, v);
-        rows++;
-        slots += f;
-    }
+    uint32_t row_n = 0, slot_n = 0, live_n = 0;   // of the lane's rows (one lane of the row counts)
+    for_rows(graphs, sp, sl, [&](const GraphDev& g, uint32_t, bool mine, uint32_t v) {
+        const uint32_t f = mine ? gp(g.fill)[v] : 0u, s = mine ? gp(g.row_ptr)[v] : 0u;
+        const bool one = mine && sublane() == 0, few = f <= GROUP_ROW;
+        const uint32_t live = compact_row_group(g, mine && few, v, s, f);
+        row_n += one;
+        slot_n += one ? f : 0u;
+        live_n += one && few ? live : 0u;
+        each_row(ballot(one && !few), v, [&](uint32_t x) {
+            const uint32_t n = compact_row_wave(g, x);
+            live_n += lane() == 0 ? n : 0u;
+        });
+    });
+    rows += wave_sum32(row_n);
+    slots += wave_sum32(slot_n);
+    live_total += wave_sum32(live_n);
     if (lane() != 0) live_total = rows = slots = 0;
     block_add64(totals, T_LIVE_SLOTS, live_total);
     block_add64(totals, T_SWEEP_ROWS + 0, rows);
@@ -1025,6 +1095,50 @@ __device__ __forceinline__ void rebuild_hub_block(const GraphDev& g, uint32_t v,
     __syncthreads();
 }
 
+// A hub row by one wavefront, into its own 1024-bin tile.
+__device__ __forceinline__ void rebuild_hub_wave(const GraphDev& g, uint32_t v, uint32_t* b) {
+    const uint32_t s = gp(g.row_ptr)[v], e = s + gp(g.fill)[v];
+    for (uint32_t t = lane(); t < HIST_BINS; t += WAVE) b[t] = 0;
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t base = s; base < e; base += ROW_UNROLL * WAVE) {
+        uint32_t nb[ROW_UNROLL], c[ROW_UNROLL];
+#pragma unroll
+        for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+            const uint32_t j = base + u * WAVE + lane();
+            nb[u] = j < e ? gp(g.col)[j] : INVALID;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < ROW_UNROLL; u++)
+            c[u] = (nb[u] != INVALID && nb[u] < g.n) ? color_of(gp(g.word)[nb[u]]) : 0;
+#pragma unroll
+        for (uint32_t u = 0; u < ROW_UNROLL; u++)
+            if (c[u] != 0 && c[u] <= HIST_BINS) atomicAdd(&b[c[u] - 1], 1u);
+    }
+    __builtin_amdgcn_wave_barrier();
+    SGC_G uint32_t* dst = gp(g.hist) + (size_t)gp(g.hd_map)[v] * HIST_BINS;
+    for (uint32_t t = lane(); t < HIST_BINS; t += WAVE) dst[t] = b[t];
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Bitmap rows of at most GROUP_ROW slots, 16 lanes each: the lane's row of
+// vertex v, if `mine` (slots [s, s + f)).
+__device__ __forceinline__ void rebuild_bitmap_group(const GraphDev& g, bool mine, uint32_t v, uint32_t s, uint32_t f) {
+    uint32_t nb[ROW_UNROLL];
+    uint64_t bm = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t j = u * GROUP + sublane();
+        nb[u] = mine && j < f ? gp(g.col)[s + j] : INVALID;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t c = (nb[u] != INVALID && nb[u] < g.n) ? color_of(gp(g.word)[nb[u]]) : 0;
+        if (c != 0 && c <= 64) bm |= 1ull << (c - 1);
+    }
+    for (uint32_t o = GROUP / 2; o > 0; o >>= 1) bm |= __shfl_xor(bm, o);
+    if (mine && sublane() == 0) gp(g.bitmap)[v] = bm;
+}
+
 // A bitmap row: the OR of its live neighbours' colours <= 64 (one wavefront,
 // or the whole block for a long row).
 template <bool kBlock>
@@ -1086,41 +1200,20 @@ __global__ __launch_bounds__(256) void k_rebuild(const GraphDev* __restrict__ gr
         else rebuild_hub_block(g, v, hd, &bins[0][0]);
     }
     uint32_t* b = bins[threadIdx.x / WAVE];
-    const uint32_t total = sweep_small(sl, sp.total);
-    for (uint32_t k = wave_id(); k < total; k += wave_count()) {
-        uint32_t gid, v;
-        sp.locate(small_item(sl, k), gid, v);
-        const GraphDev& g = graphs[gid];
-        const uint32_t hd = gp(g.hd_map)[v];
-        if (hd != INVALID && !exact_hist) continue;
-        const uint32_t s = gp(g.row_ptr)[v], e = s + gp(g.fill)[v];
-        rows++;
-        slots += e - s;
-        if (hd == INVALID) {
-            rebuild_bitmap<false>(g, v);
-            continue;
-        }
-        for (uint32_t t = lane(); t < HIST_BINS; t += WAVE) b[t] = 0;
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t base = s; base < e; base += ROW_UNROLL * WAVE) {
-            uint32_t nb[ROW_UNROLL], c[ROW_UNROLL];
-#pragma unroll
-            for (uint32_t u = 0; u < ROW_UNROLL; u++) {
-                const uint32_t j = base + u * WAVE + lane();
-                nb[u] = j < e ? gp(g.col)[j] : INVALID;
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < ROW_UNROLL; u++)
-                c[u] = (nb[u] != INVALID && nb[u] < g.n) ? color_of(gp(g.word)[nb[u]]) : 0;
-#pragma unroll
-            for (uint32_t u = 0; u < ROW_UNROLL; u++)
-                if (c[u] != 0 && c[u] <= HIST_BINS) atomicAdd(&b[c[u] - 1], 1u);
-        }
-        __builtin_amdgcn_wave_barrier();
-        SGC_G uint32_t* dst = gp(g.hist) + (size_t)hd * HIST_BINS;
-        for (uint32_t t = lane(); t < HIST_BINS; t += WAVE) dst[t] = b[t];
-        __builtin_amdgcn_wave_barrier();
-    }
+    uint32_t row_n = 0, slot_n = 0;   // of the lane's rows (one lane of the row counts)
+    for_rows(graphs, sp, sl, [&](const GraphDev& g, uint32_t, bool mine, uint32_t v) {
+        const uint32_t hd = mine ? gp(g.hd_map)[v] : INVALID;
+        const uint32_t f = mine ? gp(g.fill)[v] : 0u, s = mine ? gp(g.row_ptr)[v] : 0u;
+        const bool todo = mine && (hd == INVALID || exact_hist), one = todo && sublane() == 0;
+        const bool few = hd == INVALID && f <= GROUP_ROW;
+        row_n += one;
+        slot_n += one ? f : 0u;
+        rebuild_bitmap_group(g, todo && few, v, s, f);
+        each_row(ballot(one && !few && hd == INVALID), v, [&](uint32_t x) { rebuild_bitmap<false>(g, x); });
+        each_row(ballot(one && hd != INVALID), v, [&](uint32_t x) { rebuild_hub_wave(g, x, b); });
+    });
+    rows += wave_sum32(row_n);
+    slots += wave_sum32(slot_n);
     if (lane() != 0) rows = slots = 0;
     block_add64(totals, T_SWEEP_ROWS + 1, rows);
     block_add64(totals, T_SWEEP_SLOTS + 1, slots);
@@ -1379,6 +1472,30 @@ __device__ __forceinline__ uint32_t tier1_vertex_block(const GraphDev& g, uint32
     return 1;
 }
 
+// Whether tier1_vertex would repair the lane's coloured vertex v (colour own),
+// if `mine`: 16 lanes to a row of at most GROUP_ROW slots, reads only.
+__device__ __forceinline__ bool tier1_hit_group(const GraphDev& g, bool mine, uint32_t v, uint32_t s, uint32_t f,
+                                                uint32_t own, uint32_t deg) {
+    uint32_t nb[ROW_UNROLL];
+    bool hit = false;
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t j = u * GROUP + sublane();
+        nb[u] = mine && j < f ? ld(&g.col[s + j]) : INVALID;
+    }
+    uint32_t c[ROW_UNROLL];
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++)
+        c[u] = (nb[u] != INVALID && nb[u] < g.n) ? color_of(ld(&g.word[nb[u]])) : 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++)
+        if (c[u] != 0 && c[u] == own) {
+            const uint32_t d = gp(g.deg0)[nb[u]];
+            hit |= (deg < d) || (deg == d && v < nb[u]);   // pi(v) < pi(nb)
+        }
+    return group_bits(ballot(hit)) != 0;
+}
+
 __global__ __launch_bounds__(256) void k_tier1_elem(const GraphDev* __restrict__ graphs, Space sp, SweepList sl,
                                                     int fresh, uint64_t* totals) {
     __shared__ uint32_t presence[BLOCK / WAVE][PRESENCE_WORDS];
@@ -1397,21 +1514,30 @@ __global__ __launch_bounds__(256) void k_tier1_elem(const GraphDev* __restrict__
         }
     }
     uint32_t cnt = 0, cur_gid = 0xFFFFFFFFu;
-    const uint32_t total = sweep_small(sl, sp.total);
-    for (uint32_t k = wave_id(); k < total; k += wave_count()) {
-        uint32_t gid, v;
-        sp.locate(small_item(sl, k), gid, v);
+    uint32_t row_n = 0, slot_n = 0;   // of the lane's rows (one lane of the row counts)
+    for_rows(graphs, sp, sl, [&](const GraphDev& g, uint32_t gid, bool mine, uint32_t v) {
         if (gid != cur_gid) {
             if (cnt && lane() == 0) add32(&graphs[cur_gid].ctr[C_CONFLICTS], cnt);
             cnt = 0;
             cur_gid = gid;
         }
-        const GraphDev& g = graphs[gid];
-        rows++;
-        slots += gp(g.fill)[v];
-        cnt += tier1_vertex(g, v, presence[threadIdx.x / WAVE], fresh);
-    }
+        const uint32_t f = mine ? ld(&g.fill[v]) : 0u, s = mine ? gp(g.row_ptr)[v] : 0u;
+        const uint32_t own = mine ? color_of(ld(&g.word[v])) : 0u, deg = mine ? gp(g.deg0)[v] : 0u;
+        const bool one = mine && sublane() == 0;
+        row_n += one;
+        slot_n += one ? f : 0u;
+        // Most listed rows turn out conflict-free: 16 lanes find that, and the
+        // wavefront takes only the others (and uncoloured vertices, longer
+        // rows, and every row where the live degree decides).
+        const bool quick = mine && f <= GROUP_ROW && own != 0 && !(g.flags & ABL_LIVE_DEGREE);
+        const bool hit = tier1_hit_group(g, quick, v, s, f, own, deg);
+        each_row(ballot(one && (!quick || hit)), v, [&](uint32_t x) {
+            cnt += tier1_vertex(g, x, presence[threadIdx.x / WAVE], fresh);
+        });
+    });
     if (cnt && lane() == 0) add32(&graphs[cur_gid].ctr[C_CONFLICTS], cnt);
+    rows += wave_sum32(row_n);
+    slots += wave_sum32(slot_n);
     if (lane() != 0) rows = slots = 0;
     block_add64(totals, T_SWEEP_ROWS + 2, rows);
     block_add64(totals, T_SWEEP_SLOTS + 2, slots);
@@ -1876,6 +2002,26 @@ __device__ __forceinline__ uint32_t t2_row(const GraphDev& g, uint32_t v) {
     return kBlock ? block_sum32(bad) : wave_sum32(bad);
 }
 
+// The same for rows of at most GROUP_ROW slots, 16 lanes each: the bad slots of
+// the lane's row of vertex v, if `mine` (slots [s, s + f)).
+__device__ __forceinline__ uint32_t t2_row_group(const GraphDev& g, bool mine, uint32_t v, uint32_t s, uint32_t f) {
+    const uint32_t cv = mine ? color_of(gp(g.word)[v]) : 0u;
+    uint32_t nb[ROW_UNROLL], bad = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++) {
+        const uint32_t j = u * GROUP + sublane();
+        nb[u] = mine && j < f ? gp(g.col)[s + j] : INVALID;
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < ROW_UNROLL; u++)
+        if (nb[u] != INVALID && nb[u] < g.n && nb[u] != v) {
+            const uint32_t cn = color_of(gp(g.word)[nb[u]]);
+            bad += (cv == 0 || cn == 0 || cv == cn);
+        }
+    for (uint32_t o = GROUP / 2; o > 0; o >>= 1) bad += __shfl_xor(bad, o);
+    return bad;
+}
+
 // Tier-2 has work iff some row slot joins an uncoloured endpoint or two
 // endpoints of one colour (A/src/streamgc.cu:1190-1218 then change nothing).
 // A vertex found with a bad slot keeps its mark, so the next check counts it
@@ -1898,19 +2044,24 @@ __global__ __launch_bounds__(256) void k_t2_check(const GraphDev* __restrict__ g
             }
         }
     }
-    const uint32_t total = sweep_small(sl, sp.total);
-    for (uint32_t k = wave_id(); k < total; k += wave_count()) {
-        uint32_t gid, v;
-        sp.locate(small_item(sl, k), gid, v);
-        const GraphDev& g = graphs[gid];
-        const uint32_t bad = t2_row<false>(g, v);
-        rows++;
-        slots += gp(g.fill)[v];
-        if (bad && lane() == 0) {
+    uint32_t row_n = 0, slot_n = 0;   // of the lane's rows (one lane of the row counts)
+    for_rows(graphs, sp, sl, [&](const GraphDev& g, uint32_t, bool mine, uint32_t v) {
+        const uint32_t f = mine ? gp(g.fill)[v] : 0u, s = mine ? gp(g.row_ptr)[v] : 0u;
+        const bool one = mine && sublane() == 0, few = f <= GROUP_ROW;
+        row_n += one;
+        slot_n += one ? f : 0u;
+        uint32_t bad = t2_row_group(g, mine && few, v, s, f);
+        each_row(ballot(one && !few), v, [&](uint32_t x) {
+            const uint32_t n = t2_row<false>(g, x);
+            if (one && x == v) bad = n;
+        });
+        if (one && bad) {
             add32(&g.ctr[C_T2BAD], bad);
             if (g.dirty) gp(g.dirty)[(size_t)M_T2 * g.dstride + v] = 1;
         }
-    }
+    });
+    rows += wave_sum32(row_n);
+    slots += wave_sum32(slot_n);
     if (lane() != 0) rows = slots = 0;
     block_add64(totals, T_SWEEP_ROWS + 3, rows);
     block_add64(totals, T_SWEEP_SLOTS + 3, slots);
