@@ -31,10 +31,7 @@ constexpr uint32_t WAVE = 64;
 constexpr uint32_t ROW_UNROLL = 4;
 // An insert's or delete's scan of its two rows loads ROW_UNROLL 64-slot
 // chunks of each per round trip, and SCAN_CHUNKS of the one row left once the
-// other is done: a hub row's long search takes SCAN_CHUNKS x 64 slots per trip.
-// 8 rather than 16: every trip runs the code of all SCAN_CHUNKS chunks, and
-// the shorter trips made the per-update kernel 8% faster on a 4M-vertex
-// power-law graph although hub rows take twice as many of them.
+// other is done; while more than that is left of a row, long_search takes over.
 constexpr uint32_t SCAN_CHUNKS = 8;
 constexpr int MAX_CAS_RETRIES = 64;          // recolour CAS retries before leaving it to repair
 // Ablation flags carried by the descriptors (the values of SGC_ABL_* in streamgc.h).
@@ -133,6 +130,13 @@ __device__ __forceinline__ uint64_t wave_min64(uint64_t x) {
 }
 __device__ __forceinline__ uint32_t wave_sum32(uint32_t x) {
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_min32(uint32_t x) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t y = __shfl_xor(x, o);
+        x = y < x ? y : x;
+    }
     return x;
 }
 __device__ __forceinline__ uint32_t wave_max32(uint32_t x) {
@@ -319,6 +323,60 @@ __device__ __forceinline__ void on_neighbor_recolor(const GraphDev& g, uint32_t 
 }
 
 // ---------------------------------------------------------------- slack-CSR rows
+// The first slot of [b, end) that holds `want` (or, INSERT, is free), or
+// INVALID; eq: it holds want.  free: the first free slot passed, if none was
+// before (deletes).  For rows with more than LONG_SCAN slots to go: one trip
+// loads 8 pairs of slots a lane, 1,024 slots, where a trip of scan_pair takes
+// 512.  A hub row's scan is one chain of such trips (1.2-1.5 us each), and the
+// longest chain ended the launch: of 32,768 updates of the 4M-vertex power-law
+// graph one read 37.5K slots in 90 of the launch's 91 us, now in 41.  16 pairs
+// take 215 registers in the per-update kernel, which leaves it 2 wavefronts a
+// SIMD instead of 3.
+constexpr uint32_t LONG_SCAN = SCAN_CHUNKS * WAVE;
+template <bool INSERT>
+__device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, uint32_t end, uint32_t want, bool& eq,
+                                                uint32_t& free) {
+    constexpr uint32_t PAIRS = 8, STEP = 2 * WAVE;
+    const uint64_t none = want ? 0ull : 1ull | 1ull << 32;   // neither want nor free
+    const auto first_of = [](uint32_t m, uint32_t j) {       // the wave's first slot of the lanes' masks
+        uint32_t at = INVALID;
+        if (m) {
+            const uint32_t k = (uint32_t)__builtin_ctz(m);
+            at = j + (k >> 1) * STEP + (k & 1u);
+        }
+        return wave_min32(at);
+    };
+    // pairs start at even slots (the slot array is padded to a whole pair)
+    for (uint32_t a = b & ~1u; a < end; a += PAIRS * STEP) {
+        const uint32_t j = a + 2 * lane(), left = end > j ? end - j : 0u;
+        uint64_t p[PAIRS];
+#pragma unroll
+        for (uint32_t q = 0; q < PAIRS; q++)
+            p[q] = q * STEP < left ? ld((const uint64_t*)(g.col + j + q * STEP)) : none;
+        uint32_t ok = j < b ? ~1u : ~0u;   // a slot before b, a slot past the end
+        if (left % STEP == 1 && left / STEP < PAIRS) ok &= ~(2u << (2 * (left / STEP)));
+        uint32_t hit = 0, hole = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < PAIRS; q++)
+            hit |= (uint32_t)((uint32_t)p[q] == want) << (2 * q) | (uint32_t)((uint32_t)(p[q] >> 32) == want) << (2 * q + 1);
+        hit &= ok;
+        if (INSERT || free == INVALID) {
+#pragma unroll
+            for (uint32_t q = 0; q < PAIRS; q++)
+                hole |= (uint32_t)((uint32_t)p[q] == INVALID) << (2 * q) |
+                        (uint32_t)((uint32_t)(p[q] >> 32) == INVALID) << (2 * q + 1);
+            hole &= ok;
+            if (!INSERT && ballot(hole != 0)) free = first_of(hole, j);
+        }
+        if (ballot((INSERT ? hit | hole : hit) != 0)) {
+            const uint32_t at = first_of(INSERT ? hit | hole : hit, j);
+            eq = !INSERT || (ballot(hit != 0) != 0 && first_of(hit, j) == at);
+            return at;
+        }
+    }
+    return INVALID;
+}
+
 // A/src/kernels/local_update.cu:12-39.  First slot that is free (claimed by
 // CAS) or already holds nb.  Returns the slots scanned; a full row appends to
 // the overflow buffer (entries past capacity are dropped, the counter keeps
@@ -331,6 +389,11 @@ __device__ __forceinline__ void on_neighbor_recolor(const GraphDev& g, uint32_t 
 // Whether slots [from, end) hold nb (wave-uniform).
 __device__ __forceinline__ bool row_holds(const GraphDev& g, uint32_t nb, uint32_t from, uint32_t end) {
     constexpr uint32_t CH = SCAN_CHUNKS;   // 64-slot chunks per round trip
+    if (from < end && end - from > LONG_SCAN) {
+        bool eq;
+        uint32_t unused = 0;
+        return long_search<false>(g, from, end, nb, eq, unused) != INVALID;
+    }
     bool dup = false;
     for (uint32_t base = from; base < end && !dup; base += CH * WAVE) {
         uint32_t val[CH];
@@ -507,24 +570,39 @@ __device__ __forceinline__ void scan_pair(const GraphDev& g, bool run0, uint32_t
     while (run0 || run1) {
         c0 = c1 = INVALID;
         eq0 = eq1 = false;
-        uint32_t per0, per1;
-        if (run0 && run1 && end0 - b0 <= WAVE && end1 - b1 <= WAVE) {
-            // Both rows end within one chunk: a trip of two chunks (light
-            // rows, the common case, run far fewer instructions).
-            per0 = per1 = 1;
-            trip(std::integral_constant<uint32_t, 2>{}, per0, per1);
+        const bool long0 = run0 && end0 - b0 > LONG_SCAN, long1 = run1 && end1 - b1 > LONG_SCAN;
+        if (long0 || long1) {
+            // one row of the two (one copy of the code), the other at the next turn
+            bool eq = false;
+            uint32_t fr = long0 ? free0 : free1;
+            const uint32_t at = long_search<INSERT>(g, long0 ? b0 : b1, long0 ? end0 : end1, long0 ? nb0 : nb1, eq, fr);
+            if (long0) {
+                c0 = at, eq0 = eq, free0 = fr;
+                run0 = at != INVALID;
+            } else {
+                c1 = at, eq1 = eq, free1 = fr;
+                run1 = at != INVALID;
+            }
         } else {
-            per0 = run0 ? (run1 ? ROW_UNROLL : CH) : 0;
-            per1 = run1 ? (run0 ? ROW_UNROLL : CH) : 0;
-            trip(std::integral_constant<uint32_t, CH>{}, per0, per1);
-        }
-        if (run0 && c0 == INVALID) {
-            b0 += per0 * WAVE;
-            run0 = b0 < end0;
-        }
-        if (run1 && c1 == INVALID) {
-            b1 += per1 * WAVE;
-            run1 = b1 < end1;
+            uint32_t per0, per1;
+            if (run0 && run1 && end0 - b0 <= WAVE && end1 - b1 <= WAVE) {
+                // Both rows end within one chunk: a trip of two chunks (light
+                // rows, the common case, run far fewer instructions).
+                per0 = per1 = 1;
+                trip(std::integral_constant<uint32_t, 2>{}, per0, per1);
+            } else {
+                per0 = run0 ? (run1 ? ROW_UNROLL : CH) : 0;
+                per1 = run1 ? (run0 ? ROW_UNROLL : CH) : 0;
+                trip(std::integral_constant<uint32_t, CH>{}, per0, per1);
+            }
+            if (run0 && c0 == INVALID) {
+                b0 += per0 * WAVE;
+                run0 = b0 < end0;
+            }
+            if (run1 && c1 == INVALID) {
+                b1 += per1 * WAVE;
+                run1 = b1 < end1;
+            }
         }
         if (INSERT && c0 != INVALID && eq0) {   // the neighbour is there already
             pos0 = c0 - s0 + 1;
@@ -681,6 +759,37 @@ __device__ __forceinline__ void color_fresh(const GraphDev& g, uint32_t x, uint3
     mark_neighbors(g, x, 0, c);
 }
 
+// The colours of an insert whose slots are written; cu and cv were read after
+// that: a recolour of an endpoint after the read sees the new slot and marks
+// the other endpoint itself, so no second read is needed.
+__device__ __forceinline__ void insert_colours(const GraphDev& g, uint32_t u, uint32_t v, uint32_t hu, uint32_t hv,
+                                               uint16_t cu, uint16_t cv, WaveAcc& acc) {
+    if (cu == 0 || cv == 0) {   // first colouring of an endpoint (:90-101)
+        if (lane() == 0) {
+            mark(g, u, D_BITS | D_STATUS);
+            mark(g, v, D_BITS | D_STATUS);
+        }
+        const uint32_t wu = bcast0(ld(&g.word[u]));
+        if (color_of(wu) == 0) color_fresh(g, u, wu);
+        const uint32_t wv = bcast0(ld(&g.word[v]));
+        if (color_of(wv) == 0) {
+            on_new_neighbor(g, v, hv, color_of(bcast0(ld(&g.word[u]))));
+            color_fresh(g, v, wv);
+        }
+        cu = color_of(bcast0(ld(&g.word[u])));
+        cv = color_of(bcast0(ld(&g.word[v])));
+    }
+    on_new_neighbor(g, u, hu, cv);
+    on_new_neighbor(g, v, hv, cu);
+    if (cu == cv) {   // same colour (or both uncoloured): the sweeps look again whatever happens here
+        if (lane() == 0) {
+            mark(g, u, D_STATUS);
+            mark(g, v, D_STATUS);
+        }
+        if (cu != 0) recolor(g, pi_less(g, u, v) ? u : v, acc);
+    }
+}
+
 // One update, A/src/kernels/local_update.cu:71-146.  The reads each step
 // needs are issued together (row bounds, histogram rows, words), and both rows
 // are scanned and claimed in the same round trips (scan_pair).  A vertex word
@@ -824,33 +933,7 @@ __device__ __forceinline__ void apply_update(const GraphDev& g, uint32_t u, uint
                 mark(g, v, held_v);
             }
         }
-        if (cu == 0 || cv == 0) {   // first colouring of an endpoint (:90-101)
-            if (lane() == 0) {
-                mark(g, u, D_BITS | D_STATUS);
-                mark(g, v, D_BITS | D_STATUS);
-            }
-            const uint32_t wu = bcast0(ld(&g.word[u]));
-            if (color_of(wu) == 0) color_fresh(g, u, wu);
-            const uint32_t wv = bcast0(ld(&g.word[v]));
-            if (color_of(wv) == 0) {
-                on_new_neighbor(g, v, hv, color_of(bcast0(ld(&g.word[u]))));
-                color_fresh(g, v, wv);
-            }
-            cu = color_of(bcast0(ld(&g.word[u])));
-            cv = color_of(bcast0(ld(&g.word[v])));
-        }
-        on_new_neighbor(g, u, hu, cv);
-        on_new_neighbor(g, v, hv, cu);
-        // The colours were read after both slots were written: a recolour of
-        // an endpoint after that read sees the new slot and marks the other
-        // endpoint itself, so no second read is needed.
-        if (cu == cv) {   // same colour (or both uncoloured): the sweeps look again whatever happens here
-            if (lane() == 0) {
-                mark(g, u, D_STATUS);
-                mark(g, v, D_STATUS);
-            }
-            if (cu != 0) recolor(g, pi_less(g, u, v) ? u : v, acc);
-        }
+        insert_colours(g, u, v, hu, hv, cu, cv, acc);
         acc.scan += p;
     } else {
         const uint32_t ru = ld(&g.word[u]), rv = ld(&g.word[v]);

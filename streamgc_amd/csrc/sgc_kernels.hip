@@ -328,6 +328,19 @@ __device__ __forceinline__ uint32_t key_hash(uint64_t k, uint32_t mask) {
     return (uint32_t)k & mask;
 }
 
+// The listed edges of a batch by the longer of their two rows: those with more
+// than HEAVY_FILL filled slots (the long scans, which start first) from the
+// front of `heads`, the light ones (four to a wavefront, apply_quad) from its
+// end.  The line lies where 8 lanes still scan a row as fast as the chip needs:
+// 262K updates of 64 graphs of 2^10..2^15 vertices take 291 us with light
+// edges up to 64 slots, 257 up to 256 and 213 up to 1,024; a 131,072-vertex
+// mesh and the 4M-vertex power-law graph take the same with all three.
+constexpr uint32_t HEAVY_FILL = 1024;
+__device__ __forceinline__ uint32_t head_entry(const uint32_t* __restrict__ heads, uint32_t cap, uint32_t j,
+                                               uint32_t heavy) {
+    return j < heavy ? heads[j] : heads[cap - 1 - (j - heavy)];
+}
+
 __global__ __launch_bounds__(256) void k_group_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ head,
                                                      uint32_t size, uint32_t* __restrict__ nheads) {
     if (blockIdx.x == 0 && threadIdx.x < 2) nheads[threadIdx.x] = 0;
@@ -357,13 +370,9 @@ __device__ __forceinline__ uint32_t group_slot(uint64_t* __restrict__ keys, uint
 // once (the update that inserted the key adds its slot; an update whose key
 // found no slot is listed alone, position | GROUP_SINGLE): the per-update
 // kernel then runs one wavefront per edge.  Records that change nothing
-// (out-of-range vertex, other kinds) are not listed.  Edges with an endpoint
-// row filled past HEAVY_FILL slots (the long scans) go to the front of the
-// list, the others to the back, so that the long ones start first and the
-// short ones fill in behind them.  Each block appends its entries with one
-// atomic per list end; nheads = [front, back] counts.
+// (out-of-range vertex, other kinds) are not listed.  Each block appends its
+// entries with one atomic per list end; nheads = [heavy, light] counts.
 constexpr uint32_t GROUP_SINGLE = 0x80000000u;
-constexpr uint32_t HEAVY_FILL = 1024;
 
 __global__ __launch_bounds__(256) void k_group_link(const GraphDev* __restrict__ graphs,
                                                     const uint32_t* __restrict__ gbase,
@@ -401,15 +410,15 @@ __global__ __launch_bounds__(256) void k_group_link(const GraphDev* __restrict__
             }
             gp(next)[i] = prev;
         }
-        uint32_t nf, nb;
-        const uint32_t af = block_scan32(entry != NONE && heavy ? 1u : 0u, &nf);
-        const uint32_t ab = block_scan32(entry != NONE && !heavy ? 1u : 0u, &nb);
-        if (threadIdx.x == 0) {
-            block_at[0] = nf ? add32(&nheads[0], nf) : 0u;
-            block_at[1] = nb ? add32(&nheads[1], nb) : 0u;
+        uint32_t total;   // both counts in one scan, 16 bits each (a block has at most 256)
+        const uint32_t before = block_scan32(entry == NONE ? 0u : heavy ? 1u : 1u << 16, &total);
+        if (threadIdx.x < 2) {
+            const uint32_t mine = threadIdx.x ? total >> 16 : total & 0xFFFFu;
+            block_at[threadIdx.x] = mine ? add32(&nheads[threadIdx.x], mine) : 0u;
         }
         __syncthreads();
-        if (entry != NONE) gp(heads)[heavy ? block_at[0] + af : cap - 1 - (block_at[1] + ab)] = entry;
+        if (entry != NONE)
+            gp(heads)[heavy ? block_at[0] + (before & 0xFFFFu) : cap - 1 - (block_at[1] + (before >> 16))] = entry;
         __syncthreads();
     }
 }
@@ -436,9 +445,9 @@ __global__ __launch_bounds__(256) void k_group_pack(const uint4* __restrict__ up
                                                     const uint32_t* __restrict__ nheads, uint4* __restrict__ pack,
                                                     const uint32_t* __restrict__ dyn) {
     if (dyn) upd += dyn[0];
-    const uint32_t nf = nheads[0], n = nf + nheads[1];
+    const uint32_t nh = nheads[0], n = nh + nheads[1];
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-        const uint32_t e = j < nf ? heads[j] : heads[cap - 1 - (j - nf)];
+        const uint32_t e = head_entry(heads, cap, j, nh);
         uint32_t p0 = NONE, p1 = NONE, p2 = NONE, p3 = NONE;
         bool more = false;
         if (e & GROUP_SINGLE) {
@@ -487,7 +496,298 @@ __device__ __forceinline__ void apply_record(const GraphDev* __restrict__ graphs
     apply_rec(graphs, upd[i], multi, acc, hint);
 }
 
-__global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ graphs,
+// ---- four light edges to a wavefront
+// An edge with short rows keeps a wavefront's lanes mostly idle, and the chip
+// runs out of wavefront slots long before it runs out of anything else: the
+// update is a chain of some eight dependent loads and atomics.  So a
+// wavefront takes four such edges at once, 16 lanes each: 8 lanes on the first
+// endpoint's row (x = u) and 8 on the second's (x = v), each lane holding its
+// own endpoint's values.  One lane a row (the lead) claims the slot and writes
+// the marks, the bitmap and the histogram.  Selecting a colour stays the whole
+// wavefront's work, for one edge after another.  The steps of an update and
+// their order are apply_update's.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t x) {   // a lane exchange within 16 lanes
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t other8(uint32_t x) { return dpp<0x128>(x); }   // the other endpoint's (row_ror:8)
+__device__ __forceinline__ uint32_t min8(uint32_t x) {   // over the 8 lanes: quad_perm 1 and 2 apart, row_half_mirror
+    uint32_t y = dpp<0xB1>(x);
+    x = y < x ? y : x;
+    y = dpp<0x4E>(x);
+    x = y < x ? y : x;
+    y = dpp<0x141>(x);
+    return y < x ? y : x;
+}
+__device__ __forceinline__ uint32_t lead8(uint32_t x) {   // the 8 lanes' first lane's
+    const uint32_t q = dpp<0x00>(x), m = dpp<0x141>(q);
+    return (lane() & 4u) ? m : q;
+}
+
+constexpr uint32_t PAIR_UNROLL = 8, PAIR_SLOTS = 16 * PAIR_UNROLL;   // slots of a row loaded in one round trip
+
+struct LaneCounts {   // of the lane's own edges; summed when the wavefront ends
+    uint32_t updates = 0, scan = 0, hd = 0, ovf = 0, grouped = 0;
+};
+
+// The packed records of the lane's edge (`mine`: record k in lane k of its 16)
+// in stream order, for the edges of graph g that take part (act).
+__device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const uint4& mine, WaveAcc& acc,
+                                           LaneCounts& n) {
+    const uint32_t l8 = lane() & 7u;
+    const bool second = (lane() & 8u) != 0, lead = l8 == 0;
+    uint32_t s = 0, cap = 0, hd = INVALID;   // the row's first slot, its slots, the histogram row
+    bool sticky = false;
+    // The RowHint of a delete that removed both copies (held_x = its x, or INVALID).
+    uint32_t held_x = INVALID, held = 0, freed = 0, own = 0, seen = 0;
+    for (uint32_t k = 0; k < GROUP_PACK; k++) {
+        const int from_lane = (int)((lane() & 48u) + k);
+        const uint32_t rx = (uint32_t)__shfl((int)mine.x, from_lane), ry = (uint32_t)__shfl((int)mine.y, from_lane);
+        const bool ins = (__shfl((int)mine.z, from_lane) & 0xFF) == 0;
+        const bool on = act && rx != PACK_NONE;
+        if (!ballot(on)) break;
+        const uint32_t x = second ? ry : rx, y = second ? rx : ry;
+        const bool hinted = on && ins && held_x == x;
+        uint32_t f = 0, w = 0;
+        uint64_t bits = ~0ull;
+        if (on && !hinted) {
+            if (held_x != INVALID && lead) mark(g, held_x, held);
+            held_x = INVALID;
+            s = gp(g.row_ptr)[x];
+            cap = gp(g.row_ptr)[x + 1] - s;
+            hd = gp(g.hd_map)[x];
+            sticky = g.dirty && gp(g.dirty)[(size_t)M_STICKY * g.dstride + x];
+            f = ld(&g.fill[x]);
+            if (!ins) {
+                w = ld(&g.word[x]);
+                bits = ld(&g.bitmap[x]);
+            }
+        }
+        uint32_t pos = 0, pf = 0, open = INVALID;   // as scan_pair's pos, pf, free (here from the row's start)
+        bool had = false, run = on;
+        if (ballot(hinted)) {   // claim the slots the delete left
+            uint32_t old = 0, raised = 0;
+            if (hinted && lead) {
+                old = cas32(&g.col[freed], INVALID, y);
+                raised = max32(&g.fill[x], freed - s + 1);
+            }
+            old = lead8(old);
+            raised = lead8(raised);
+            if (hinted) {
+                if (freed == own) held &= ~D_ROW;
+                if (old == INVALID) {
+                    pos = freed - s + 1;
+                    pf = raised;
+                    run = false;
+                } else {   // another wavefront took the slot
+                    held |= D_ROW;
+                    f = ld(&g.fill[x]);
+                }
+            }
+        }
+        const bool scanned = run;
+        uint32_t from = 0;   // slots before it were passed
+        while (ballot(run)) {   // (from grows with every trip of a row still running)
+            // pairs of slots from the even slot at or before `from` (the slot array holds whole pairs)
+            const uint32_t a = (s + from) & ~1u, j = a + 2 * l8, left = run && s + f > j ? s + f - j : 0u;
+            const uint32_t next = a + PAIR_SLOTS - s;
+            const uint64_t none = y ? 0ull : 1ull | 1ull << 32;   // neither y nor free
+            uint64_t p[PAIR_UNROLL];
+#pragma unroll
+            for (uint32_t q = 0; q < PAIR_UNROLL; q++)
+                p[q] = 16 * q < left ? ld((const uint64_t*)(g.col + j + 16 * q)) : none;
+            uint32_t ok = j < s + from ? ~1u : ~0u;   // a slot before `from`, a slot past the fill
+            if (left % 16 == 1 && left / 16 < PAIR_UNROLL) ok &= ~(2u << (2 * (left / 16)));
+            uint32_t is_y = 0, is_free = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < PAIR_UNROLL; q++) {
+                const uint32_t lo = (uint32_t)p[q], hi = (uint32_t)(p[q] >> 32);
+                is_y |= (uint32_t)(lo == y) << (2 * q) | (uint32_t)(hi == y) << (2 * q + 1);
+                is_free |= (uint32_t)(lo == INVALID) << (2 * q) | (uint32_t)(hi == INVALID) << (2 * q + 1);
+            }
+            is_y &= ok;
+            is_free &= ok;
+            const uint32_t ky = is_y ? (uint32_t)__builtin_ctz(is_y) : 0u;
+            const uint32_t kf = is_free ? (uint32_t)__builtin_ctz(is_free) : 0u;
+            uint32_t eq = is_y ? j + 16 * (ky >> 1) + (ky & 1u) - s : INVALID;
+            uint32_t fr = is_free ? j + 16 * (kf >> 1) + (kf & 1u) - s : INVALID;
+            eq = min8(eq);
+            fr = min8(fr);
+            open = fr < open ? fr : open;
+            bool claim = false;
+            uint32_t at = 0;
+            if (run && ins) {   // the first slot that is free or holds y; past the fill every slot is free
+                uint32_t first = eq < fr ? eq : fr;
+                if (first == INVALID && next >= f) first = f;
+                if (first == INVALID) {
+                    from = next;
+                } else if (first == eq) {
+                    pos = eq + 1;
+                    had = true;
+                    run = false;
+                } else if (first >= cap) {
+                    run = false;   // the row is full
+                } else {
+                    claim = true;
+                    at = first;
+                }
+            } else if (run) {
+                claim = eq != INVALID;
+                at = eq;
+                if (!claim) {
+                    from = next;
+                    run = from < f;
+                }
+            }
+            uint32_t old = 0, raised = 0;
+            if (claim && lead) {
+                old = cas32(&g.col[s + at], ins ? INVALID : y, ins ? y : INVALID);
+                if (ins) raised = max32(&g.fill[x], at + 1);
+            }
+            old = lead8(old);
+            raised = lead8(raised);
+            if (claim) {
+                const bool won = old == (ins ? INVALID : y);
+                if (won || (ins && old == y)) {
+                    pos = at + 1;
+                    pf = ins && won ? raised : 0u;
+                    had = ins && !won;
+                    run = false;
+                } else {   // another wavefront took the slot: go on after it
+                    from = at + 1;
+                    if (ins) {
+                        const uint32_t now = ld(&g.fill[x]);
+                        f = now > from ? now : from;
+                    } else {
+                        run = from < f;
+                    }
+                }
+            }
+        }
+        const uint32_t pos2 = other8(pos);
+        // ---- delete: marks, histogram, colour reduction
+        const uint32_t c1 = color_of(w), o1 = other8(c1);
+        bool reduce = false;
+        if (on && !ins) {
+            const uint32_t m = (pos ? D_ROW : 0u) | ((hd == INVALID) == (pos != 0) ? D_BITS : 0u);
+            if (pos && pos2) {
+                held_x = x;
+                held = m;
+                own = s + pos - 1;
+                freed = s + (open < pos - 1 ? open : pos - 1);
+                seen = o1;
+            } else if (lead) {
+                mark(g, x, m);
+            }
+            if (lead) {
+                if (hd != INVALID && o1 != 0 && o1 <= HIST_BINS)
+                    add32(&g.hist[(size_t)hd * HIST_BINS + o1 - 1], 0xFFFFFFFFu);
+                n.scan += pos ? pos : f;
+            }
+            // try_reduce, up to where it selects a colour
+            reduce = c1 != 0 && o1 < c1 &&
+                     !(hd == INVALID && ~bits && (uint32_t)__builtin_ctzll(~bits) + 1u >= c1);
+        }
+        for (uint64_t todo = ballot(reduce && lead); todo; todo &= todo - 1) {   // u before v
+            const uint32_t i = (uint32_t)__builtin_ctzll(todo), z = __builtin_amdgcn_readlane(x, i);
+            if (find_color(g, z) < __builtin_amdgcn_readlane(c1, i)) recolor(g, z, acc);
+        }
+        // ---- insert: a second copy of the edge, overflow, marks, colours
+        if (ballot(on && ins)) {
+            const bool add = on && ins;
+            const bool had2 = other8(had) != 0, sticky2 = other8(sticky) != 0, scanned2 = other8(scanned) != 0;
+            const uint32_t tail = pf > pos ? pf - pos : 0u, tail2 = other8(tail);
+            // (apply_update says which row has to be searched for a second copy)
+            bool dup = false, look = false;
+            if (add && !(sticky && sticky2) && !(hinted && !scanned && !scanned2)) {
+                if (pos && pos2) {
+                    dup = had != had2;
+                    look = !had && !had2 && tail && (second ? tail < tail2 : tail <= tail2);
+                } else {
+                    look = pos && tail;
+                }
+            }
+            for (uint32_t b = pos; ballot(look); b += 8 * PAIR_UNROLL) {
+                uint32_t val[PAIR_UNROLL];
+                bool any = false;
+#pragma unroll
+                for (uint32_t q = 0; q < PAIR_UNROLL; q++) {
+                    const uint32_t j = b + 8 * q + l8;
+                    val[q] = look && j < pf ? ld(&g.col[s + j]) : INVALID;
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < PAIR_UNROLL; q++) any |= val[q] == y;
+                const bool found = ((ballot(any) >> (lane() & 56u)) & 0xFFu) != 0;
+                dup |= look && found;
+                look = look && !found && b + 8 * PAIR_UNROLL < pf;
+            }
+            const bool dup2 = other8(dup) != 0;
+            uint32_t now = 0;
+            if (add) {
+                if (lead) {
+                    if (!second && (dup || dup2)) {
+                        add32(&g.ctr[C_ASYM], 1u);
+                        mark_sticky(g, x);
+                        mark_sticky(g, y);
+                    }
+                    if (!pos) {   // overflow (finish_insert)
+                        add32(&g.ctr[C_ASYM], 1u);
+                        const uint32_t at = add32(&g.ctr[C_OVF], 1u);
+                        if (at < g.ovf_cap) {
+                            st(&g.ovf[2 * (size_t)at], x);
+                            st(&g.ovf[2 * (size_t)at + 1], y);
+                        }
+                        mark_sticky(g, x);
+                        mark_sticky(g, y);
+                        n.ovf++;
+                    }
+                    n.scan += pos ? pos : cap;
+                    if (had) mark(g, x, D_BITS);
+                }
+                now = ld(&g.word[x]);
+            }
+            const uint32_t c = color_of(now), o = other8(c);
+            const bool odd = add && (c == 0 || o == 0 || c == o);   // colours to select or to settle
+            if (hinted) {   // the delete's marks, less what the re-insert undid
+                if (o == seen) held &= ~D_BITS;
+                if (lead) mark(g, x, held);
+                held_x = INVALID;
+            }
+            if (add && !odd && lead) {   // on_new_neighbor
+                if (o <= 64) or64(&g.bitmap[x], 1ull << (o - 1));
+                if (hd != INVALID && o <= HIST_BINS) add32(&g.hist[(size_t)hd * HIST_BINS + o - 1], 1u);
+            }
+            for (uint64_t todo = ballot(odd && lead && !second); todo; todo &= todo - 1) {
+                const uint32_t i = (uint32_t)__builtin_ctzll(todo);
+                insert_colours(g, __builtin_amdgcn_readlane(x, i), __builtin_amdgcn_readlane(y, i),
+                               __builtin_amdgcn_readlane(hd, i), __builtin_amdgcn_readlane(hd, i + 8),
+                               (uint16_t)__builtin_amdgcn_readlane(c, i), (uint16_t)__builtin_amdgcn_readlane(o, i),
+                               acc);
+            }
+        }
+        if (on && lead) {
+            n.hd += hd != INVALID;
+            if (!second) {
+                n.updates++;
+                n.grouped += k > 0;
+            }
+        }
+    }
+    if (act && held_x != INVALID && lead) mark(g, held_x, held);   // marks of a last delete
+}
+
+// One wavefront per heavy edge of the batch, then one per four light ones.  Up
+// to APPLY_SPREAD light edges take a wavefront each: the chip runs some 3,000
+// wavefronts of this kernel (3 a SIMD, for its 168 registers) and one edge's
+// chain is shorter alone (1,338 light edges of a 65,536-vertex R-MAT graph,
+// launch: 37 us alone, 45 us by fours).  Launch times with one edge a wavefront
+// and scans of 512 slots a trip / now: 32,768 updates of a 131,072-vertex mesh
+// 56 / 37 us, of the 4M-vertex power-law graph 100 / 60, of dense growth on a
+// 2^18-vertex R-MAT graph 157 / 108; 4,099 updates of the 65,536-vertex one
+// 56 / 37; a pool's 262K updates 308 / 213.  Bound: the chain of dependent
+// gathers and atomics of an edge, over the wavefronts the registers allow.
+constexpr uint32_t APPLY_SPREAD = 4096;
+__global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict__ graphs,
                                                     const uint4* __restrict__ upd, uint32_t count, int multi,
                                                     const uint32_t* __restrict__ ghead,
                                                     const uint32_t* __restrict__ gnext,
@@ -506,51 +806,89 @@ __global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ 
         acc.flush(totals);
         return;
     }
-    // One wavefront per edge of the batch: its updates in stream order.  The
-    // records come from the edge's packed 64-byte line (lanes 0..3 load one
-    // each), or, for a group longer than the line, from its list (head, then
-    // next links): repeatedly the record at the smallest position above the
-    // last one applied.
-    const uint32_t nf = nheads[0], n = nf + nheads[1];
-    for (uint32_t j = wave_id(); j < n; j += wave_count()) {
-        uint4 mine = make_uint4(PACK_NONE, PACK_WALK, 0u, 0u);
-        if (pack && lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
-        const bool walk = __builtin_amdgcn_readlane(mine.x, 0) == PACK_NONE &&
-                          __builtin_amdgcn_readlane(mine.y, 0) == PACK_WALK;
-        uint32_t h = NONE;
-        bool single = false;
-        if (walk) {
-            const uint32_t e = j < nf ? heads[j] : heads[cap - 1 - (j - nf)];   // long scans first
-            single = (e & GROUP_SINGLE) != 0;
-            h = single ? e & ~GROUP_SINGLE : gp(ghead)[e];
-        }
-        RowHint hint;   // a delete's slots for the same edge's re-insert (a last delete's marks wait in it)
-        hint.valid = false;
-        uint32_t applied = 0, last = 0, last_g = 0;
-        for (;;) {
-            uint4 r;
-            if (!walk) {
-                if (applied == GROUP_PACK) break;
-                r = make_uint4(__builtin_amdgcn_readlane(mine.x, applied), __builtin_amdgcn_readlane(mine.y, applied),
-                               __builtin_amdgcn_readlane(mine.z, applied), __builtin_amdgcn_readlane(mine.w, applied));
-                if (r.x == PACK_NONE) break;
-            } else if (single) {
-                if (applied) break;
-                r = upd[h];
-            } else {
-                uint32_t best = NONE;
-                for (uint32_t k2 = h; k2 != NONE; k2 = gp(gnext)[k2])
-                    if ((applied == 0 || k2 > last) && (best == NONE || k2 < best)) best = k2;
-                if (best == NONE) break;
-                r = upd[best];
-                last = best;
+    // An edge's updates in stream order.  The records come from the edge's
+    // packed 64-byte line (one lane each), or, for a group longer than the
+    // line, from its list (head, then next links): repeatedly the record at
+    // the smallest position above the last one applied.
+    const uint32_t nh = nheads[0], nl = nheads[1];
+    const uint32_t per = pack && nl > APPLY_SPREAD ? GROUPS : 1u;
+    const uint32_t jobs = nh + (nl + per - 1) / per;
+    LaneCounts lanes;
+    for (uint32_t job = wave_id(); job < jobs; job += wave_count()) {
+        uint32_t j0 = job, whole = 1u;   // first edge; which of the (up to four) edges the whole wavefront takes
+        if (per > 1 && job >= nh) {
+            j0 = nh + (job - nh) * per;
+            const uint32_t j = j0 + lane() / GROUP;
+            const bool have = j < nh + nl;
+            uint4 mine = make_uint4(PACK_NONE, PACK_END, 0u, 0u);
+            if (have && sublane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + sublane()];
+            const int first = (int)(lane() & 48u);
+            const uint32_t x = (uint32_t)__shfl((int)mine.x, first), y = (uint32_t)__shfl((int)mine.y, first);
+            const uint32_t gid = multi ? (uint32_t)__shfl((int)mine.w, first) : 0u;
+            // groups longer than the line and self-loops take the whole wavefront, and ablations
+            bool quad = have && x != PACK_NONE && x != y;
+            whole = 0;
+            for (uint64_t pend = ballot(quad); pend;) {   // one graph after another
+                const uint32_t g0 = __builtin_amdgcn_readlane(gid, (uint32_t)__builtin_ctzll(pend));
+                const bool in = quad && gid == g0;
+                pend &= ~ballot(in);
+                const GraphDev g = graphs[g0];
+                if (g.flags) quad = quad && !in;
+                else apply_quad(g, in, mine, acc, lanes);
             }
-            apply_rec(graphs, r, multi, acc, &hint);
-            last_g = r.w;
-            applied++;
+            const uint64_t left = ballot(have && !quad && sublane() == 0);
+            for (uint32_t i = 0; i < GROUPS; i++) whole |= (uint32_t)((left >> (GROUP * i)) & 1u) << i;
         }
-        if (hint.valid) hint_release(graphs[multi ? last_g : 0u], &hint);   // marks of a last delete
-        grouped += applied ? applied - 1 : 0;
+        for (; whole; whole &= whole - 1) {
+            const uint32_t j = j0 + (uint32_t)__builtin_ctz(whole);
+            uint4 mine = make_uint4(PACK_NONE, PACK_WALK, 0u, 0u);
+            if (pack && lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
+            const bool walk = __builtin_amdgcn_readlane(mine.x, 0) == PACK_NONE &&
+                              __builtin_amdgcn_readlane(mine.y, 0) == PACK_WALK;
+            uint32_t h = NONE;
+            bool single = false;
+            if (walk) {
+                const uint32_t e = head_entry(heads, cap, j, nh);
+                single = (e & GROUP_SINGLE) != 0;
+                h = single ? e & ~GROUP_SINGLE : gp(ghead)[e];
+            }
+            RowHint hint;   // a delete's slots for the same edge's re-insert (a last delete's marks wait in it)
+            hint.valid = false;
+            uint32_t applied = 0, last = 0, last_g = 0;
+            for (;;) {
+                uint4 r;
+                if (!walk) {
+                    if (applied == GROUP_PACK) break;
+                    r = make_uint4(__builtin_amdgcn_readlane(mine.x, applied),
+                                   __builtin_amdgcn_readlane(mine.y, applied),
+                                   __builtin_amdgcn_readlane(mine.z, applied),
+                                   __builtin_amdgcn_readlane(mine.w, applied));
+                    if (r.x == PACK_NONE) break;
+                } else if (single) {
+                    if (applied) break;
+                    r = upd[h];
+                } else {
+                    uint32_t best = NONE;
+                    for (uint32_t k2 = h; k2 != NONE; k2 = gp(gnext)[k2])
+                        if ((applied == 0 || k2 > last) && (best == NONE || k2 < best)) best = k2;
+                    if (best == NONE) break;
+                    r = upd[best];
+                    last = best;
+                }
+                apply_rec(graphs, r, multi, acc, &hint);
+                last_g = r.w;
+                applied++;
+            }
+            if (hint.valid) hint_release(graphs[multi ? last_g : 0u], &hint);   // marks of a last delete
+            grouped += applied ? applied - 1 : 0;
+        }
+    }
+    if (per > 1) {
+        acc.updates += wave_sum32(lanes.updates);
+        acc.scan += wave_sum32(lanes.scan);
+        acc.hd += wave_sum32(lanes.hd);
+        acc.ovf += wave_sum32(lanes.ovf);
+        grouped += wave_sum32(lanes.grouped);
     }
     acc.flush(totals);
     if (grouped && totals && lane() == 0) tot_add(totals, T_GROUPED, grouped);
