@@ -68,8 +68,8 @@ __device__ __forceinline__ uint32_t big_item(const SweepList& sl, uint32_t k) { 
 // The front rows of a sweep set (or every row) over the grid's wavefronts.
 // Rows are short -- 6 slots on a mesh, 17 on a social graph -- and a row is one
 // chain of dependent loads (list entry, row bounds, slots, neighbours' words),
-// so a wavefront takes four rows at a time, 16 lanes each; a grid with more
-// wavefronts than rows takes one each.  A full sweep of 4.0M rows and 69M live
+// so a wavefront takes up to four rows at a time, 16 lanes each, as many as its
+// share of the rows.  A full sweep of 4.0M rows and 69M live
 // slots, one row a wavefront / four: compaction 1,180 / 324 us, rebuild 2,200 /
 // 1,137 us, Tier-1 3,513 / 1,071 us (what is left is the gather of 69M
 // neighbour words).  body(g, gid, mine, v) runs with g wave-uniform (rows of several graphs: one graph after another): mine says
@@ -84,7 +84,8 @@ template <class F>
 __device__ __forceinline__ void for_rows(const GraphDev* __restrict__ graphs, const Space& sp, const SweepList& sl,
                                          F&& body) {
     const uint32_t total = sweep_small(sl, sp.total);
-    const uint32_t per = total > wave_count() ? GROUPS : 1u, mine_of = lane() / GROUP;
+    const uint32_t fair = (total + wave_count() - 1) / wave_count();   // rows a wavefront
+    const uint32_t per = fair < 1 ? 1u : fair < GROUPS ? fair : GROUPS, mine_of = lane() / GROUP;
     for (uint32_t k0 = wave_id() * per; k0 < total; k0 += wave_count() * per) {
         const bool have = mine_of < per && k0 + mine_of < total;
         uint32_t gid = 0, v = 0;
@@ -1204,38 +1205,76 @@ __global__ __launch_bounds__(256) void k_snapshot(const GraphDev* __restrict__ g
 // changes: a live value moves to w + (live lanes before it); a slot whose
 // value moved and that lies past the chunk's new write front is freed (a
 // later chunk may refill it, in program order).
-// One long row, all threads of the block: windows of 1024 slots (4
-// consecutive slots per thread), a block prefix of the live counts, then the
-// moves.  Writes of a window land below its end, reads of the next window
-// start at its end.  Returns the live count; the row's fill becomes it.
+// A block barrier for data in LDS: outstanding global loads and stores go on
+// across it (__syncthreads waits for them).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One long row, all threads of the block, windows of COMPACT_WINDOW slots: the
+// live slots of each 64-slot chunk are counted by ballot, one lane of each
+// wavefront adds up a chunk's place, and the live values move there.  A value
+// moves down or stays, and only to slots below its window's end, which every
+// wavefront has read by then (it counted them), so the next window's loads are
+// in flight meanwhile; slots past the live ones are freed once, at the end.
+// Returns the live count; the row's fill becomes it.
+// A long row is one block's chain of windows, and the longest row ends the
+// launch; with 1,024 slots a window and every store waited for, a window took
+// 1.1 us.  Compaction after 32,768 updates of dense growth on a 2^18-vertex
+// R-MAT graph (longest row 32K slots) 44 -> 28 us, of churn on the 4M-vertex
+// power-law graph (14K slots) 19.8 -> 16.
+constexpr uint32_t COMPACT_PER = 16, COMPACT_WINDOW = COMPACT_PER * BLOCK;
 __device__ __forceinline__ uint32_t compact_row_block(const GraphDev& g, uint32_t v) {
+    static_assert(COMPACT_PER * (BLOCK / WAVE) == WAVE, "one lane a chunk");
+    __shared__ uint32_t part[2][WAVE];   // live slots of the window's chunks, in slot order
+    const uint64_t lt_mask = (1ull << lane()) - 1ull;
     const uint32_t s = gp(g.row_ptr)[v], e = s + gp(g.fill)[v];
-    uint32_t w = s;
-    for (uint32_t base = s; base < e; base += 4 * BLOCK) {
-        const uint32_t j0 = base + 4 * threadIdx.x;
-        uint32_t val[4], cnt = 0;
+    const uint32_t wv = bcast0(threadIdx.x / WAVE);
+    uint32_t w = s, buf = 0, next[COMPACT_PER];
 #pragma unroll
-        for (uint32_t q = 0; q < 4; q++) {
-            val[q] = j0 + q < e ? gp(g.col)[j0 + q] : INVALID;
-            cnt += val[q] != INVALID;
-        }
-        uint32_t total = 0;
-        uint32_t pos = w + block_scan32(cnt, &total);
-        const uint32_t w_after = w + total;
-#pragma unroll
-        for (uint32_t q = 0; q < 4; q++) {
-            const uint32_t j = j0 + q;
-            if (val[q] == INVALID) continue;
-            if (pos != j) {
-                gp(g.col)[pos] = val[q];
-                if (j >= w_after) gp(g.col)[j] = INVALID;
-            }
-            pos++;
-        }
-        w = w_after;
-        __syncthreads();
+    for (uint32_t q = 0; q < COMPACT_PER; q++) {
+        const uint32_t j = s + q * BLOCK + threadIdx.x;
+        next[q] = j < e ? gp(g.col)[j] : INVALID;
     }
+    for (uint32_t base = s; base < e; base += COMPACT_WINDOW, buf ^= 1u) {
+        uint32_t val[COMPACT_PER];
+#pragma unroll
+        for (uint32_t q = 0; q < COMPACT_PER; q++) val[q] = next[q];
+        uint32_t mine = 0;   // lane q: the live slots of the wavefront's chunk q
+#pragma unroll
+        for (uint32_t q = 0; q < COMPACT_PER; q++) {
+            const uint32_t n = (uint32_t)__builtin_popcountll(ballot(val[q] != INVALID));
+            mine = lane() == q ? n : mine;
+        }
+        if (lane() < COMPACT_PER) part[buf][lane() * (BLOCK / WAVE) + wv] = mine;
+#pragma unroll
+        for (uint32_t q = 0; q < COMPACT_PER; q++) {
+            const uint32_t j = base + COMPACT_WINDOW + q * BLOCK + threadIdx.x;
+            next[q] = j < e ? gp(g.col)[j] : INVALID;
+        }
+        lds_barrier();   // (the other buffer was read before the barrier of the window before)
+        const uint32_t x = part[buf][lane()];
+        uint32_t inc = x;
+        for (uint32_t d = 1; d < WAVE; d <<= 1) {
+            const uint32_t y = __shfl_up(inc, d);
+            if (lane() >= d) inc += y;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < COMPACT_PER; q++) {
+            const uint32_t j = base + q * BLOCK + threadIdx.x;
+            const bool live = val[q] != INVALID;
+            const uint32_t pos = w + __builtin_amdgcn_readlane(inc - x, q * (BLOCK / WAVE) + wv) +
+                                 (uint32_t)__builtin_popcountll(ballot(live) & lt_mask);
+            if (live && pos != j) gp(g.col)[pos] = val[q];
+        }
+        w += __builtin_amdgcn_readlane(inc, WAVE - 1);
+    }
+    __syncthreads();   // the moves are done: free what lies past the live slots
+    for (uint32_t j = w + threadIdx.x; j < e; j += BLOCK) gp(g.col)[j] = INVALID;
     if (threadIdx.x == 0) gp(g.fill)[v] = w - s;
+    __syncthreads();   // (part is used again)
     return w - s;
 }
 
@@ -1305,10 +1344,12 @@ __device__ __forceinline__ void drain_prep_graph(const GraphDev* __restrict__ gr
     c[C_DRAIN_FAILED] = 0;
 }
 
+// (256, 8): with more than 64 registers only 7 of a CU's 8 blocks of the usual
+// grid run at once, and a full sweep waits for the eighth (327 -> 526 us).
 // prep_ng > 0: block 0 also takes the drain's counter snapshot of the
 // active graphs (k_drain_prep), which the drain launched next reads;
 // compaction touches none of those counters.
-__global__ __launch_bounds__(256) void k_compact(const GraphDev* __restrict__ graphs, Space sp, SweepList sl,
+__global__ __launch_bounds__(256, 8) void k_compact(const GraphDev* __restrict__ graphs, Space sp, SweepList sl,
                                                  uint64_t* totals, uint32_t prep_ng,
                                                  const uint32_t* __restrict__ prep_active) {
     if (blockIdx.x == 0)
