@@ -323,18 +323,16 @@ __device__ __forceinline__ void on_neighbor_recolor(const GraphDev& g, uint32_t 
 }
 
 // ---------------------------------------------------------------- slack-CSR rows
-// The first slot of [b, end) that holds `want` (or, INSERT, is free), or
-// INVALID; eq: it holds want.  free: the first free slot passed, if none was
-// before (deletes).  For rows with more than LONG_SCAN slots to go: one trip
-// loads 8 pairs of slots a lane, 1,024 slots, where a trip of scan_pair takes
-// 512.  A hub row's scan is one chain of such trips (1.2-1.5 us each), and the
-// longest chain ended the launch: of 32,768 updates of the 4M-vertex power-law
-// graph one read 37.5K slots in 90 of the launch's 91 us, now in 41.  16 pairs
-// take 215 registers in the per-update kernel, which leaves it 2 wavefronts a
-// SIMD instead of 3.
+// The first slot of [b, end) that holds `want`, or INVALID.  free: the first
+// free slot passed, if none was before.  For rows with more than LONG_SCAN
+// slots to go: one trip loads 8 pairs of slots a lane, 1,024 slots, where a
+// trip of scan_pair takes 512.  A hub row's scan is one chain of such trips
+// (1.2-1.5 us each), and the longest chain ended the launch: of 32,768 updates
+// of the 4M-vertex power-law graph one read 37.5K slots in 90 of the launch's
+// 91 us, now in 41.  16 pairs take 215 registers in the per-update kernel,
+// which leaves it 2 wavefronts a SIMD instead of 3.
 constexpr uint32_t LONG_SCAN = SCAN_CHUNKS * WAVE;
-template <bool INSERT>
-__device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, uint32_t end, uint32_t want, bool& eq,
+__device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, uint32_t end, uint32_t want,
                                                 uint32_t& free) {
     constexpr uint32_t PAIRS = 8, STEP = 2 * WAVE;
     const uint64_t none = want ? 0ull : 1ull | 1ull << 32;   // neither want nor free
@@ -360,27 +358,19 @@ __device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, u
         for (uint32_t q = 0; q < PAIRS; q++)
             hit |= (uint32_t)((uint32_t)p[q] == want) << (2 * q) | (uint32_t)((uint32_t)(p[q] >> 32) == want) << (2 * q + 1);
         hit &= ok;
-        if (INSERT || free == INVALID) {
+        if (free == INVALID) {
 #pragma unroll
             for (uint32_t q = 0; q < PAIRS; q++)
                 hole |= (uint32_t)((uint32_t)p[q] == INVALID) << (2 * q) |
                         (uint32_t)((uint32_t)(p[q] >> 32) == INVALID) << (2 * q + 1);
             hole &= ok;
-            if (!INSERT && ballot(hole != 0)) free = first_of(hole, j);
+            if (ballot(hole != 0)) free = first_of(hole, j);
         }
-        if (ballot((INSERT ? hit | hole : hit) != 0)) {
-            const uint32_t at = first_of(INSERT ? hit | hole : hit, j);
-            eq = !INSERT || (ballot(hit != 0) != 0 && first_of(hit, j) == at);
-            return at;
-        }
+        if (ballot(hit != 0)) return first_of(hit, j);
     }
     return INVALID;
 }
 
-// A/src/kernels/local_update.cu:12-39.  First slot that is free (claimed by
-// CAS) or already holds nb.  Returns the slots scanned; a full row appends to
-// the overflow buffer (entries past capacity are dropped, the counter keeps
-// counting) or, with overflow disabled, reports failure.
 // An insert that lands in a hole may duplicate a copy further along the row
 // (the first-free-or-equal scan meets the hole first,
 // A/src/kernels/local_update.cu:12-40); a later delete then removes one copy
@@ -390,9 +380,8 @@ __device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, u
 __device__ __forceinline__ bool row_holds(const GraphDev& g, uint32_t nb, uint32_t from, uint32_t end) {
     constexpr uint32_t CH = SCAN_CHUNKS;   // 64-slot chunks per round trip
     if (from < end && end - from > LONG_SCAN) {
-        bool eq;
         uint32_t unused = 0;
-        return long_search<false>(g, from, end, nb, eq, unused) != INVALID;
+        return long_search(g, from, end, nb, unused) != INVALID;
     }
     bool dup = false;
     for (uint32_t base = from; base < end && !dup; base += CH * WAVE) {
@@ -515,6 +504,12 @@ __device__ __forceinline__ void mark_neighbors(const GraphDev& g, uint32_t v, ui
 // pf = the fill before an insert's raise when this wave wrote the slot, else 0;
 // had = an insert found the neighbour in the row already; free = the first
 // free slot a delete's scan passed (absolute index, INVALID: none).
+// A delete's rows with more than LONG_SCAN slots to go are scanned by
+// long_search.  Inserts keep to the short trips: a hub's inserts then come to
+// their colour choices one after another, as far as their edges lie in its row.
+// All at once they cost colours (the 4M-vertex power-law graph coloured from
+// its edges in launches of 256: 84-87 colours in 6 runs, 81-83 in 8 with the
+// short trips; the sequential replay has 83).
 template <bool INSERT>
 __device__ __forceinline__ void scan_pair(const GraphDev& g, bool run0, uint32_t x0, uint32_t nb0, uint32_t s0,
                                           uint32_t end0, bool run1, uint32_t x1, uint32_t nb1, uint32_t s1,
@@ -570,17 +565,16 @@ __device__ __forceinline__ void scan_pair(const GraphDev& g, bool run0, uint32_t
     while (run0 || run1) {
         c0 = c1 = INVALID;
         eq0 = eq1 = false;
-        const bool long0 = run0 && end0 - b0 > LONG_SCAN, long1 = run1 && end1 - b1 > LONG_SCAN;
+        const bool long0 = !INSERT && run0 && end0 - b0 > LONG_SCAN, long1 = !INSERT && run1 && end1 - b1 > LONG_SCAN;
         if (long0 || long1) {
             // one row of the two (one copy of the code), the other at the next turn
-            bool eq = false;
             uint32_t fr = long0 ? free0 : free1;
-            const uint32_t at = long_search<INSERT>(g, long0 ? b0 : b1, long0 ? end0 : end1, long0 ? nb0 : nb1, eq, fr);
+            const uint32_t at = long_search(g, long0 ? b0 : b1, long0 ? end0 : end1, long0 ? nb0 : nb1, fr);
             if (long0) {
-                c0 = at, eq0 = eq, free0 = fr;
+                c0 = at, free0 = fr;
                 run0 = at != INVALID;
             } else {
-                c1 = at, eq1 = eq, free1 = fr;
+                c1 = at, free1 = fr;
                 run1 = at != INVALID;
             }
         } else {

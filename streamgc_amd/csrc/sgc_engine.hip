@@ -269,8 +269,9 @@ struct sgc_pool {
     uint32_t rev_cap = 0;
     uint32_t* d_t2_items = nullptr;       // (graph, vertex, old colour) recoloured by the host Tier-2
     size_t t2_items_cap = 0;
-    uint32_t* d_list = nullptr;           // sweep worklist (virtual vertex ids)
-    uint32_t* d_list_count = nullptr;
+    uint32_t* d_list = nullptr;           // sweep worklists (virtual vertex ids): the current sweep's, a later one's
+    uint32_t* d_list_count = nullptr;     // their lengths
+    uint32_t ahead = NO_KIND;             // the later sweep whose worklist is built already
     uint32_t list_cap = 0;
     uint32_t ng = 0, V = 0;               // slots in use, vertices
     uint32_t act_n = 0, act_V = 0;        // active graphs and their vertices
@@ -456,7 +457,7 @@ struct sgc_pool {
             if (d_list) (void)hipFree(d_list);
             d_list = nullptr;
             list_cap = 0;
-            if (e == hipSuccess) e = hipMalloc((void**)&d_list, list_words(V, max_graphs) * 4);
+            if (e == hipSuccess) e = hipMalloc((void**)&d_list, 2 * list_words(V, max_graphs) * 4);
             if (e == hipSuccess) list_cap = V;
         }
         return e;
@@ -464,12 +465,38 @@ struct sgc_pool {
 
     // The sweep context: the vertices of the active graphs marked for sweep
     // `kind` (their marks are cleared) or sticky; every vertex without tracking.
-    hipError_t sweep(LaunchCtx& L, uint32_t kind) {
+    // `later`: the same set's sweep of that kind comes next and its worklist is
+    // built in the same launches (nothing in between may mark a vertex for it
+    // that is not sticky: compaction marks none, the drain only endpoints of
+    // overflowed edges).
+    hipError_t sweep(LaunchCtx& L, uint32_t kind, uint32_t later = NO_KIND) {
         if (!tracking()) return hipSuccess;
         L.list = d_list;
         L.list_count = d_list_count;
         L.list_cap = list_cap;
-        return timed("build_list", [&] { return launch_build_list(L, kind, d_list, list_cap, d_list_count); });
+        if (kind == ahead) {
+            L.list += second_list();
+            L.list_count += 2;
+            ahead = NO_KIND;
+            return hipSuccess;
+        }
+        ahead = later;
+        return timed("build_list", [&] {
+            return launch_build_list(L, kind, d_list, list_cap, d_list_count, later, second_list());
+        });
+    }
+    size_t second_list() const { return list_words(list_cap, max_graphs); }
+    // The sweep that follows an epoch's compaction and drain over the same
+    // graphs, or NO_KIND where it is not the same for all of them: Tier-1 with
+    // live colours, or the rebuild.
+    uint32_t next_sweep(const std::vector<uint32_t>& gids, bool repair) const {
+        if (!repair) return M_BITS;
+        uint32_t live = 0;
+        for (uint32_t g : gids) {
+            if (gs[g].cfg.max_repair_iters == 0) return NO_KIND;   // no Tier-1 sweep
+            live += fresh_level(g) == 2;
+        }
+        return live == gids.size() ? (uint32_t)M_CHECK : live == 0 ? (uint32_t)M_BITS : NO_KIND;
     }
     // All sweeps must visit every vertex of graph gid (its state changed from the host).
     hipError_t mark_all(uint32_t gid) {
@@ -533,6 +560,7 @@ struct sgc_pool {
     int device_tier2(const std::vector<uint32_t>& list, std::vector<uint32_t>& host_jobs, std::vector<uint32_t>& ran);
     int publish(const std::vector<uint32_t>& gids);
     int read_drain(const std::vector<uint32_t>& gids);
+    void drain_stats(const std::vector<uint32_t>& gids);
     int max_colors(const std::vector<uint32_t>& gids);
 
     // ------------------------------------------------------------ batched runs
@@ -772,12 +800,15 @@ int sgc_pool::apply(const sgc_edge_update* upd, uint32_t count, bool on_device, 
 int sgc_pool::read_drain(const std::vector<uint32_t>& gids) {
     hipError_t e = read_ctr();
     if (e != hipSuccess) return hip_fail(e, "counters");
+    drain_stats(gids);
+    return SGC_OK;
+}
+void sgc_pool::drain_stats(const std::vector<uint32_t>& gids) {
     for (uint32_t g : gids) {
         gs[g].st.overflow_count = ctr(g, C_OVF_RAW);
         gs[g].st.overflow_drained = ctr(g, C_OVF_RAW) ? ctr(g, C_OVF_SNAP) : 0;
         gs[g].st.overflow_failed = ctr(g, C_DRAIN_FAILED);
     }
-    return SGC_OK;
 }
 
 // run_conflict_repair (A/src/streamgc.cu:1317-1393) for every graph of the set
@@ -815,7 +846,7 @@ int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it) {
         }
         if (e == hipSuccess) e = set_active_iterating(gids);
         LaunchCtx L = ctx(true);
-        if (e == hipSuccess) e = launch_zero_ctr(L, C_CONFLICTS);
+        if (e == hipSuccess && it > 0) e = launch_zero_ctr(L, C_CONFLICTS);   // (the drain's preparation cleared it)
         // A graph sweeps in vertex order on one wavefront (Gauss-Seidel) when
         // deterministic, or when it is small and two parallel sweeps have left
         // a few conflicts (a racy sweep over a small conflict set can chase the
@@ -1112,13 +1143,18 @@ int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<
         L = ctx(true);
     }
     LaunchCtx Lc = L;
-    if (e == hipSuccess) e = sweep(Lc, M_ROW);
+    ahead = NO_KIND;
+    if (e == hipSuccess) e = sweep(Lc, M_ROW, next_sweep(gids, repair));
     if (e == hipSuccess) e = timed("compact", [&] { return launch_compact(Lc, true); });
     uint32_t ovf_cap = 0;
     for (uint32_t g : gids) ovf_cap = std::max(ovf_cap, gs[g].cfg.overflow_capacity);
     if (e == hipSuccess) e = timed("drain", [&] { return launch_drain(L, deterministic(), ovf_cap, true); });
     if (e != hipSuccess) return hip_fail(e, "compact/drain");
-    if (out)   // drain statistics (the repair below reads the counters it needs itself)
+    // Drain statistics: the counters stay as the drain left them, and a repair
+    // reads them all after its first sweep.
+    bool swept = repair;
+    for (uint32_t g : gids) swept &= gs[g].cfg.max_repair_iters > 0;
+    if (out && !swept)
         if ((r = read_drain(gids))) return r;
     if (repair) {
         if (finish && rebuild_each_sweep()) {
@@ -1126,6 +1162,7 @@ int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<
             if (e != hipSuccess) return hip_fail(e, "rebuild");
         }
         if ((r = tier1(gids))) return r;
+        if (out && swept) drain_stats(gids);
         if ((r = tier2(gids))) return r;
         if (!deterministic()) {   // bitmaps and histograms exact again for the next updates
             e = set_active(gids);
@@ -1380,7 +1417,11 @@ int sgc_pool::batch_capture(const sgc_tuning& t, hipGraphExec_t* out) {
     const int fresh = B.all_settled ? (int)t.fresh_repair : 0;
     const bool rebuild_sweep = det || fresh < 2;
     bool serial_ok = false;   // some graph is small enough for serial sweeps
-    for (uint32_t g = 0; g < ng; g++) serial_ok |= gs[g].used && gs[g].n <= t.serial_repair;
+    bool sweeping = true;     // every graph of a round starts with a parallel Tier-1 sweep (det: a rebuild)
+    for (uint32_t g = 0; g < ng; g++) {
+        serial_ok |= gs[g].used && gs[g].n <= t.serial_repair;
+        sweeping &= !gs[g].used || gs[g].cfg.max_repair_iters > 0;
+    }
     hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "batch capture");
     e = launch_round_begin(stream, B.d_ctl, B.d_tab, B.d_inround, ng, B.d_fl, B.d_state, B.d_rg);
@@ -1396,7 +1437,10 @@ int sgc_pool::batch_capture(const sgc_tuning& t, hipGraphExec_t* out) {
     }
     LaunchCtx Lr = base;
     Lr.active = F(F_ROUND);
-    if (e == hipSuccess) e = launch_build_list(Lr, M_ROW, d_list, list_cap, d_list_count);
+    // the list of the first sweep after the drain with it (see sweep())
+    const uint32_t later = sweeping && B.sweeps > 0 ? (rebuild_sweep ? (uint32_t)M_BITS : (uint32_t)M_CHECK) : NO_KIND;
+    if (e == hipSuccess)
+        e = launch_build_list(Lr, M_ROW, d_list, list_cap, d_list_count, later, second_list());
     if (e == hipSuccess) e = launch_compact(Lr, true);
     if (e == hipSuccess) e = launch_drain(Lr, det, B.ovf_cap, true);
     for (uint32_t it = 0; it < B.sweeps && e == hipSuccess; it++) {
@@ -1406,14 +1450,24 @@ int sgc_pool::batch_capture(const sgc_tuning& t, hipGraphExec_t* out) {
             LaunchCtx Lb = base;
             Lb.active = F(F_ITER);
             Lb.gate = t1_any;
-            e = launch_build_list(Lb, M_BITS, d_list, list_cap, d_list_count);
+            if (it == 0 && later == M_BITS) {
+                Lb.list += second_list();
+                Lb.list_count += 2;
+            } else {
+                e = launch_build_list(Lb, M_BITS, d_list, list_cap, d_list_count);
+            }
             if (e == hipSuccess) e = launch_rebuild(Lb, exact_hist());
         }
         if (e == hipSuccess && !det) {
             LaunchCtx Lp = base;
             Lp.active = F(F_PAR);
             Lp.gate = t1_any;
-            e = launch_build_list(Lp, M_CHECK, d_list, list_cap, d_list_count);
+            if (it == 0 && later == M_CHECK) {
+                Lp.list += second_list();
+                Lp.list_count += 2;
+            } else {
+                e = launch_build_list(Lp, M_CHECK, d_list, list_cap, d_list_count);
+            }
             if (e == hipSuccess) e = launch_tier1(Lp, false, fresh);
         }
         if (e == hipSuccess && (det || (it >= 2 && serial_ok))) {   // parallel runs: serial after two sweeps
@@ -1823,7 +1877,7 @@ int pool_init(sgc_pool* P, uint32_t max_graphs, uint32_t batch_cap, uint32_t fla
     if (e == hipSuccess) e = hipHostMalloc(&P->h_totals, (size_t)T_STRIPES * T_STRIDE * 8);
     if (e == hipSuccess) e = hipMalloc(&P->d_batch, (size_t)batch_cap * sizeof(sgc_edge_update));
     if (e == hipSuccess) e = hipMalloc(&P->d_tmp16, 64);
-    if (e == hipSuccess) e = hipMalloc(&P->d_list_count, 8);
+    if (e == hipSuccess) e = hipMalloc(&P->d_list_count, 16);
     if (e == hipSuccess) e = hipMalloc(&P->d_rev_count, 8);
     P->eg.size = 16;
     while (P->eg.size < 2u * batch_cap) P->eg.size <<= 1;
@@ -1832,8 +1886,9 @@ int pool_init(sgc_pool* P, uint32_t max_graphs, uint32_t batch_cap, uint32_t fla
     if (e == hipSuccess) e = hipMalloc(&P->eg.head, (size_t)P->eg.size * 4);
     if (e == hipSuccess) e = hipMalloc(&P->eg.next, (size_t)batch_cap * 4);
     if (e == hipSuccess) e = hipMalloc(&P->eg.heads, (size_t)batch_cap * 4);
-    if (e == hipSuccess) e = hipMalloc(&P->eg.nheads, 8);
+    if (e == hipSuccess) e = hipMalloc(&P->eg.nheads, GROUP_WORDS * 4);
     if (e == hipSuccess) e = hipMalloc(&P->eg.pack, (size_t)batch_cap * 4 * sizeof(uint4));
+    if (e == hipSuccess) e = launch_group_clear(P->stream, P->eg);
     if (e == hipSuccess) e = hipStreamSynchronize(P->stream);
     if (e != hipSuccess) return P->hip_fail(e, "pool create");
     return SGC_OK;

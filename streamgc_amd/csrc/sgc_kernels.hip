@@ -207,12 +207,17 @@ __device__ __forceinline__ void list_tile(const GraphDev& g, uint32_t kind, uint
 }
 
 __global__ __launch_bounds__(256) void k_list_tiles(const GraphDev* __restrict__ graphs, Space sp,
-                                                    const uint32_t* __restrict__ stile, uint32_t kind,
-                                                    uint32_t long_row, uint32_t* __restrict__ tmp,
+                                                    const uint32_t* __restrict__ stile, uint32_t kind, uint32_t kind2,
+                                                    size_t second, uint32_t long_row, uint32_t* __restrict__ tmp,
                                                     uint32_t* __restrict__ tcount,
                                                     const uint32_t* __restrict__ active,
                                                     const uint32_t* __restrict__ gate) {
     if (gate && *gate == 0) return;
+    if (blockIdx.y) {   // the second list
+        kind = kind2;
+        tmp += second;
+        tcount += second;
+    }
     const uint32_t t = blockIdx.x;
     // Several graphs: their tiles laid end to end (stile = prefix of each
     // part's tile count); the part holding tile t, found by the whole block.
@@ -268,10 +273,16 @@ __global__ __launch_bounds__(256) void k_list_tiles(const GraphDev* __restrict__
 __global__ __launch_bounds__(256) void k_list_gather(const GraphDev* __restrict__ graphs, Space sp, int multi,
                                                      const uint32_t* __restrict__ tmp,
                                                      const uint32_t* __restrict__ tcount,
-                                                     uint32_t* __restrict__ list, uint32_t cap,
+                                                     uint32_t* __restrict__ list, uint32_t cap, size_t second,
                                                      uint32_t* __restrict__ count,
                                                      const uint32_t* __restrict__ active,
                                                      const uint32_t* __restrict__ gate) {
+    if (blockIdx.y) {
+        tmp += second;
+        tcount += second;
+        list += second;
+        count += 2;
+    }
     // one graph not taking part: nothing listed (several graphs: the tiles of
     // those not taking part counted nothing)
     const uint32_t gid = sp.gid ? sp.gid[0] : 0u;
@@ -337,14 +348,14 @@ __device__ __forceinline__ uint32_t key_hash(uint64_t k, uint32_t mask) {
 // edges up to 64 slots, 257 up to 256 and 213 up to 1,024; a 131,072-vertex
 // mesh and the 4M-vertex power-law graph take the same with all three.
 constexpr uint32_t HEAVY_FILL = 1024;
-__device__ __forceinline__ uint32_t head_entry(const uint32_t* __restrict__ heads, uint32_t cap, uint32_t j,
-                                               uint32_t heavy) {
-    return j < heavy ? heads[j] : heads[cap - 1 - (j - heavy)];
-}
 
+// The table is empty between batches: k_group_pack frees the slots it reads,
+// and k_apply_elem, which reads the counts that k_group_pack copied, clears the
+// ones k_group_link adds to.  A batch so needs no launch to clear the table
+// (2-4 us, and up to 12 before the next one starts when the host sets the pace).
 __global__ __launch_bounds__(256) void k_group_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ head,
                                                      uint32_t size, uint32_t* __restrict__ nheads) {
-    if (blockIdx.x == 0 && threadIdx.x < 2) nheads[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < GROUP_WORDS) nheads[threadIdx.x] = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < size; i += gridDim.x * blockDim.x) {
         gp(keys)[i] = KEY_EMPTY;
         gp(head)[i] = NONE;
@@ -372,7 +383,8 @@ __device__ __forceinline__ uint32_t group_slot(uint64_t* __restrict__ keys, uint
 // found no slot is listed alone, position | GROUP_SINGLE): the per-update
 // kernel then runs one wavefront per edge.  Records that change nothing
 // (out-of-range vertex, other kinds) are not listed.  Each block appends its
-// entries with one atomic per list end; nheads = [heavy, light] counts.
+// entries with one atomic per list end; nheads = [heavy, light] counts, and
+// k_group_pack's copy of them.
 constexpr uint32_t GROUP_SINGLE = 0x80000000u;
 
 __global__ __launch_bounds__(256) void k_group_link(const GraphDev* __restrict__ graphs,
@@ -429,7 +441,7 @@ __global__ __launch_bounds__(256) void k_group_link(const GraphDev* __restrict__
 // per-update kernel has a whole group after one load instead of walking
 // head, list links and records one dependent load after another.  Unused
 // entries are PACK_NONE records; an edge with more than GROUP_PACK updates is
-// left to the walk (its first entry says so and carries the list entry).
+// left to the walk (its first entry says so and carries the list's first position).
 constexpr uint32_t GROUP_PACK = 4;
 constexpr uint32_t PACK_NONE = 0xFFFFFFFFu;   // x of an entry with no record (a listed record has x < n)
 constexpr uint32_t PACK_END = 0, PACK_WALK = 1;   // y of such an entry
@@ -440,15 +452,17 @@ __device__ __forceinline__ void cswap(uint32_t& a, uint32_t& b) {
     b = hi;
 }
 
-__global__ __launch_bounds__(256) void k_group_pack(const uint4* __restrict__ upd, const uint32_t* __restrict__ ghead,
+__global__ __launch_bounds__(256) void k_group_pack(const uint4* __restrict__ upd, uint64_t* __restrict__ keys,
+                                                    uint32_t* __restrict__ ghead,
                                                     const uint32_t* __restrict__ gnext,
                                                     const uint32_t* __restrict__ heads, uint32_t cap,
-                                                    const uint32_t* __restrict__ nheads, uint4* __restrict__ pack,
+                                                    uint32_t* __restrict__ nheads, uint4* __restrict__ pack,
                                                     const uint32_t* __restrict__ dyn) {
     if (dyn) upd += dyn[0];
+    if (blockIdx.x == 0 && threadIdx.x < 2) nheads[2 + threadIdx.x] = nheads[threadIdx.x];
     const uint32_t nh = nheads[0], n = nh + nheads[1];
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-        const uint32_t e = head_entry(heads, cap, j, nh);
+        const uint32_t e = j < nh ? heads[j] : heads[cap - 1 - (j - nh)];
         uint32_t p0 = NONE, p1 = NONE, p2 = NONE, p3 = NONE;
         bool more = false;
         if (e & GROUP_SINGLE) {
@@ -461,8 +475,12 @@ __global__ __launch_bounds__(256) void k_group_pack(const uint4* __restrict__ up
             more = p3 != NONE && gp(gnext)[p3] != NONE;
         }
         uint4* out = pack + (size_t)j * GROUP_PACK;
+        if (!(e & GROUP_SINGLE)) {
+            gp(keys)[e] = KEY_EMPTY;
+            gp(ghead)[e] = NONE;
+        }
         if (more) {
-            out[0] = make_uint4(PACK_NONE, PACK_WALK, 0u, e);
+            out[0] = make_uint4(PACK_NONE, PACK_WALK, 0u, p0);
             continue;
         }
         cswap(p0, p1);   // sorting network for 4 (NONE sorts last)
@@ -790,10 +808,8 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
 constexpr uint32_t APPLY_SPREAD = 4096;
 __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict__ graphs,
                                                     const uint4* __restrict__ upd, uint32_t count, int multi,
-                                                    const uint32_t* __restrict__ ghead,
                                                     const uint32_t* __restrict__ gnext,
-                                                    const uint32_t* __restrict__ heads, uint32_t cap,
-                                                    const uint32_t* __restrict__ nheads,
+                                                    uint32_t* __restrict__ nheads,
                                                     const uint4* __restrict__ pack, uint64_t* totals,
                                                     const uint32_t* __restrict__ dyn) {
     WaveAcc acc;
@@ -802,17 +818,18 @@ __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict
         upd += dyn[0];
         count = dyn[1];
     }
-    if (!heads) {   // no grouping: one wavefront per position
+    if (!pack) {   // no grouping: one wavefront per position
         for (uint32_t i = wave_id(); i < count; i += wave_count()) apply_record(graphs, upd, i, multi, acc);
         acc.flush(totals);
         return;
     }
     // An edge's updates in stream order.  The records come from the edge's
     // packed 64-byte line (one lane each), or, for a group longer than the
-    // line, from its list (head, then next links): repeatedly the record at
-    // the smallest position above the last one applied.
-    const uint32_t nh = nheads[0], nl = nheads[1];
-    const uint32_t per = pack && nl > APPLY_SPREAD ? GROUPS : 1u;
+    // line, from its list: repeatedly the record at the smallest position
+    // above the last one applied.
+    const uint32_t nh = nheads[2], nl = nheads[3];
+    if (blockIdx.x == 0 && lane() < 2) nheads[lane()] = 0;   // for the next batch's k_group_link
+    const uint32_t per = nl > APPLY_SPREAD ? GROUPS : 1u;
     const uint32_t jobs = nh + (nl + per - 1) / per;
     LaneCounts lanes;
     for (uint32_t job = wave_id(); job < jobs; job += wave_count()) {
@@ -843,16 +860,10 @@ __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict
         for (; whole; whole &= whole - 1) {
             const uint32_t j = j0 + (uint32_t)__builtin_ctz(whole);
             uint4 mine = make_uint4(PACK_NONE, PACK_WALK, 0u, 0u);
-            if (pack && lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
+            if (lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
             const bool walk = __builtin_amdgcn_readlane(mine.x, 0) == PACK_NONE &&
                               __builtin_amdgcn_readlane(mine.y, 0) == PACK_WALK;
-            uint32_t h = NONE;
-            bool single = false;
-            if (walk) {
-                const uint32_t e = head_entry(heads, cap, j, nh);
-                single = (e & GROUP_SINGLE) != 0;
-                h = single ? e & ~GROUP_SINGLE : gp(ghead)[e];
-            }
+            const uint32_t h = __builtin_amdgcn_readlane(mine.w, 0);   // the list's first position
             RowHint hint;   // a delete's slots for the same edge's re-insert (a last delete's marks wait in it)
             hint.valid = false;
             uint32_t applied = 0, last = 0, last_g = 0;
@@ -865,9 +876,6 @@ __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict
                                    __builtin_amdgcn_readlane(mine.z, applied),
                                    __builtin_amdgcn_readlane(mine.w, applied));
                     if (r.x == PACK_NONE) break;
-                } else if (single) {
-                    if (applied) break;
-                    r = upd[h];
                 } else {
                     uint32_t best = NONE;
                     for (uint32_t k2 = h; k2 != NONE; k2 = gp(gnext)[k2])
@@ -1342,6 +1350,7 @@ __device__ __forceinline__ void drain_prep_graph(const GraphDev* __restrict__ gr
     if (raw > graphs[gid].ovf_cap) c[C_LOST] += raw - graphs[gid].ovf_cap;   // never buffered
     c[C_OVF] = 0;
     c[C_DRAIN_FAILED] = 0;
+    c[C_CONFLICTS] = 0;   // for the epoch's first Tier-1 sweep
 }
 
 // (256, 8): with more than 64 registers only 7 of a CU's 8 blocks of the usual
@@ -2540,34 +2549,29 @@ static inline uint32_t grid_for_waves(uint64_t waves, uint32_t waves_per_block, 
 
 hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg) {
     if (count == 0) return hipSuccess;
-    const uint32_t *head = nullptr, *next = nullptr, *heads = nullptr, *nheads = nullptr;
-    if (eg && eg->keys && count > 1) {
-        if ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->heads || !eg->nheads)
-            return hipErrorInvalidValue;
-        head = eg->head;
-        next = eg->next;
-        heads = eg->heads;
-        nheads = eg->nheads;
-    }
+    const bool group = eg && eg->keys && count > 1;
+    if (group && ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->heads || !eg->nheads || !eg->pack))
+        return hipErrorInvalidValue;
+    const EdgeGroups G = group ? *eg : EdgeGroups();
     // one-wavefront blocks: a wavefront's slot is refilled as soon as it ends
     uint32_t grid = grid_for_waves(count, 1, 4 * L.max_blocks);
-    k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, head, next, heads,
-                                               eg ? eg->next_cap : 0u, nheads, heads ? eg->pack : nullptr,
+    k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, G.next, G.nheads, G.pack,
                                                L.totals, L.dyn);
+    return hipGetLastError();
+}
+hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg) {
+    k_group_clear<<<grid_for_waves(eg.size, 4 * WAVE, 1024), 256, 0, s>>>(eg.keys, eg.head, eg.size, eg.nheads);
     return hipGetLastError();
 }
 hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg) {
     if (count <= 1 || !eg || !eg->keys) return hipSuccess;
-    if ((uint64_t)eg->size < 2ull * count || eg->next_cap < count) return hipErrorInvalidValue;
+    if ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->pack) return hipErrorInvalidValue;
     const uint32_t mask = eg->size - 1;
-    uint32_t cg = grid_for_waves(eg->size, 4 * WAVE, 1024);
-    k_group_clear<<<cg, 256, 0, L.stream>>>(eg->keys, eg->head, eg->size, eg->nheads);
     uint32_t mg = grid_for_waves(count, 4 * WAVE, 1024);
     k_group_link<<<mg, 256, 0, L.stream>>>(L.graphs, L.gbase, (const uint4*)upd, count, multi, eg->keys, eg->head,
                                            eg->next, mask, eg->heads, eg->next_cap, eg->nheads, L.dyn);
-    if (eg->pack)
-        k_group_pack<<<mg, 256, 0, L.stream>>>((const uint4*)upd, eg->head, eg->next, eg->heads, eg->next_cap,
-                                               eg->nheads, eg->pack, L.dyn);
+    k_group_pack<<<mg, 256, 0, L.stream>>>((const uint4*)upd, eg->keys, eg->head, eg->next, eg->heads, eg->next_cap,
+                                           eg->nheads, eg->pack, L.dyn);
     return hipGetLastError();
 }
 // Up to so many segments a block of wavefronts replays each, above it one
@@ -2619,8 +2623,11 @@ static inline uint32_t sweep_grid(const LaunchCtx& L) {
     return grid_for_waves(L.V, 4, L.list ? L.sweep_blocks : L.max_blocks);
 }
 static inline SweepList sweep_list(const LaunchCtx& L) { return SweepList{L.list, L.list_count, L.list_cap}; }
-hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, uint32_t cap, uint32_t* count) {
-    if (kind >= M_STICKY || cap < L.V) return hipErrorInvalidValue;
+hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, uint32_t cap, uint32_t* count,
+                             uint32_t kind2, size_t second) {
+    const bool two = kind2 != NO_KIND;
+    if (kind >= M_STICKY || (two && (kind2 >= M_STICKY || kind2 == kind || !second)) || cap < L.V)
+        return hipErrorInvalidValue;
     // Two passes over 4096-vertex tiles, each tile inside one graph (scratch
     // behind the list): one graph's own tiles, or the tiles of several graphs
     // laid end to end (L.stile, L.tiles).
@@ -2629,14 +2636,16 @@ hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, 
     if (multi && (!L.stile || tiles > list_tiles(cap, L.ng))) return hipErrorInvalidValue;
     if (tiles == 0) {
         k_zero_list_count<<<1, 1, 0, L.stream>>>(count);
+        if (two) k_zero_list_count<<<1, 1, 0, L.stream>>>(count + 2);
         return hipGetLastError();
     }
     uint32_t* tmp = list + cap;
     uint32_t* tcount = tmp + (size_t)tiles * LIST_TILE_V;
-    k_list_tiles<<<tiles, 256, 0, L.stream>>>(L.graphs, space(L), multi ? L.stile : nullptr, kind, L.long_row, tmp,
-                                              tcount, L.active, L.gate);
-    k_list_gather<<<tiles, 256, 0, L.stream>>>(L.graphs, space(L), multi ? 1 : 0, tmp, tcount, list, cap, count,
-                                               L.active, L.gate);
+    const dim3 grid(tiles, two ? 2 : 1);
+    k_list_tiles<<<grid, 256, 0, L.stream>>>(L.graphs, space(L), multi ? L.stile : nullptr, kind, kind2, second,
+                                             L.long_row, tmp, tcount, L.active, L.gate);
+    k_list_gather<<<grid, 256, 0, L.stream>>>(L.graphs, space(L), multi ? 1 : 0, tmp, tcount, list, cap, second, count,
+                                              L.active, L.gate);
     return hipGetLastError();
 }
 hipError_t launch_compact(const LaunchCtx& L, bool drain_prep) {

@@ -48,12 +48,15 @@ struct EdgeGroups {
     uint32_t* next = nullptr;
     uint32_t* heads = nullptr;    // next_cap entries: one per edge of the batch (slot, or position | 1 << 31),
                                   // long scans from the front, the others from the back
-    uint32_t* nheads = nullptr;   // device words: entries at the front, at the back
-    uint4* pack = nullptr;        // next_cap x 4 records: each listed edge's updates in stream order (or null)
+    uint32_t* nheads = nullptr;   // GROUP_WORDS device words: entries at the front, at the back, a copy of both
+    uint4* pack = nullptr;        // next_cap x 4 records: each listed edge's updates in stream order
     uint32_t size = 0;
     uint32_t next_cap = 0;
 };
 
+constexpr uint32_t GROUP_WORDS = 4;
+// Empties a new table (every batch leaves it empty).
+hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg);
 // Per-edge grouping of a parallel batch (before launch_apply with the same eg).
 hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg);
 hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg);
@@ -73,7 +76,11 @@ hipError_t launch_drain(const LaunchCtx& L, bool serial, uint32_t max_count, boo
 // Worklist of the vertices marked `kind` (or sticky).  `list` holds
 // list_words(cap, graphs) u32: the list, then the builder's scratch of
 // 4096-vertex tiles (each inside one graph, so up to one more per graph).
-hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, uint32_t cap, uint32_t* count);
+// With kind2 a second list in the same launches, its arrays `second` words
+// further on, its counts in count[2..3].
+constexpr uint32_t NO_KIND = 0xFFFFFFFFu;
+hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, uint32_t cap, uint32_t* count,
+                             uint32_t kind2 = NO_KIND, size_t second = 0);
 inline size_t list_tiles(uint32_t cap, uint32_t graphs) { return ((size_t)cap + 4095) / 4096 + graphs; }
 inline size_t list_words(uint32_t cap, uint32_t graphs) {
     const size_t tiles = list_tiles(cap, graphs);
