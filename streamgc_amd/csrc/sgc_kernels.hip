@@ -801,9 +801,9 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
 // chain is shorter alone (1,338 light edges of a 65,536-vertex R-MAT graph,
 // launch: 37 us alone, 45 us by fours).  Launch times with one edge a wavefront
 // and scans of 512 slots a trip / now: 32,768 updates of a 131,072-vertex mesh
-// 56 / 37 us, of the 4M-vertex power-law graph 100 / 60, of dense growth on a
-// 2^18-vertex R-MAT graph 157 / 108; 4,099 updates of the 65,536-vertex one
-// 56 / 37; a pool's 262K updates 308 / 213.  Bound: the chain of dependent
+// 56 / 38 us, of the 4M-vertex power-law graph 100 / 71, of dense growth on a
+// 2^18-vertex R-MAT graph 157 / 131; 4,099 updates of the 65,536-vertex one
+// 56 / 44; a pool's 262K updates 308 / 191.  Bound: the chain of dependent
 // gathers and atomics of an edge, over the wavefronts the registers allow.
 constexpr uint32_t APPLY_SPREAD = 4096;
 __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict__ graphs,
