@@ -684,7 +684,7 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
             }
         }
         const uint32_t pos2 = other8(pos);
-        // ---- delete: marks, histogram, colour reduction
+        // ---- delete: marks, histogram, whether its colour may fall
         const uint32_t c1 = color_of(w), o1 = other8(c1);
         bool reduce = false;
         if (on && !ins) {
@@ -706,10 +706,6 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
             // try_reduce, up to where it selects a colour
             reduce = c1 != 0 && o1 < c1 &&
                      !(hd == INVALID && ~bits && (uint32_t)__builtin_ctzll(~bits) + 1u >= c1);
-        }
-        for (uint64_t todo = ballot(reduce && lead); todo; todo &= todo - 1) {   // u before v
-            const uint32_t i = (uint32_t)__builtin_ctzll(todo), z = __builtin_amdgcn_readlane(x, i);
-            if (find_color(g, z) < __builtin_amdgcn_readlane(c1, i)) recolor(g, z, acc);
         }
         // ---- insert: a second copy of the edge, overflow, marks, colours
         if (ballot(on && ins)) {
@@ -783,6 +779,13 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
                                (uint16_t)__builtin_amdgcn_readlane(c, i), (uint16_t)__builtin_amdgcn_readlane(o, i),
                                acc);
             }
+        }
+        // The reductions come last: a recolour between an insert's slot writes and
+        // its read of the words would tell the new neighbour of the change, and the
+        // insert would count the new colour there a second time.
+        for (uint64_t todo = ballot(reduce && lead); todo; todo &= todo - 1) {   // u before v
+            const uint32_t i = (uint32_t)__builtin_ctzll(todo), z = __builtin_amdgcn_readlane(x, i);
+            if (find_color(g, z) < __builtin_amdgcn_readlane(c1, i)) recolor(g, z, acc);
         }
         if (on && lead) {
             n.hd += hd != INVALID;

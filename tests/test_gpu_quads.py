@@ -1,0 +1,67 @@
+"""Edges that share a vertex within one wavefront of the four-edge path.
+
+Four light edges go to a wavefront in lock-step, in the order of their records
+where every record is an edge of its own.  Each four here hold a delete at x
+that lowers x's colour and inserts that join x to a vertex with a histogram, in
+every order; fours share nothing, so words, rows (as sets: which free slot an
+insert meets depends on the order) and histograms are the sequential oracle's.
+"""
+import numpy as np
+import pytest
+
+import streamgc_amd as S
+from test_gpu_parity import _pair
+
+pytestmark = pytest.mark.gpu
+
+FOURS = 2304   # 9,216 edges: whole blocks of 256 records, and enough for the four-edge path
+LEAVES = 9     # of each histogram vertex
+
+
+def _graph():
+    """Each four's vertices: x, its neighbours a and p, two stars b0 and b1 with their leaves, and two pairs of loose
+    vertices; colours 3, 1, 1, 4 and 5, 1, and 1 and 2 (x can fall to 2 when it loses a)."""
+    size = 3 + 2 * (1 + LEAVES) + 4
+    at = np.arange(FOURS) * size
+    edges, colour = [], np.ones(FOURS * size, np.uint32)
+    for i in at.tolist():
+        edges += [(i, i + 1), (i, i + 2)]
+        for k in range(2):
+            b = i + 3 + k * (1 + LEAVES)
+            edges += [(b, b + 1 + j) for j in range(LEAVES)]
+            colour[b] = 4 + k
+        colour[[i, size + i - 3, size + i - 1]] = 3, 2, 2
+    return S.csr_from_edges(FOURS * size, edges), colour, at, size
+
+
+def _rows(csr):
+    """The slots with each row's sorted."""
+    rp, col = csr
+    row = np.repeat(np.arange(len(rp) - 1), np.diff(rp.astype(np.int64)))
+    return col[np.lexsort((col, row))]
+
+
+@pytest.mark.parametrize("threshold", [1, LEAVES - 1])   # x has a histogram as well, or a bitmap
+def test_deletes_and_inserts_at_one_vertex(threshold):
+    g, colour, at, size = _graph()
+    gpu, orc, og = _pair(g, epoch_size=1 << 20, batch_size=1 << 20, histogram_threshold=threshold,
+                         exact_histogram=True)
+    words = (colour | 1 << 16).astype(np.uint32)
+    for eng in (gpu, orc):
+        eng.set_words(words)
+        eng.finish()
+    recs = []
+    for k, x in enumerate(at.tolist()):
+        b0, b1, loose = x + 3, x + 4 + LEAVES, x + size - 4
+        gone, in0, in1, pair = (x, x + 1, 1), (x, b0, 0), (b1, x, 0), (loose, loose + 1, 0)
+        four = [[gone, in0, in1, pair], [in0, gone, pair, in1], [pair, in1, in0, gone], [in0, (x + 1, x, 1), pair,
+                (loose + 2, loose + 3, 0)]][k % 4]
+        recs += four
+    batch = S.make_updates(*(list(c) for c in zip(*recs)))
+    gpu.apply(batch)
+    orc.submit(batch["u"], batch["v"], batch["type"])
+    assert gpu.totals()["recolors"] >= FOURS
+    assert np.array_equal(gpu.words(), orc.words())
+    assert np.array_equal(_rows(gpu.csr()), _rows(orc.csr()))
+    assert np.array_equal(gpu.hist(), orc.hist())
+    assert np.all(orc.bitmaps() & ~gpu.bitmaps() == 0)   # (no neighbour's colour is missing)
