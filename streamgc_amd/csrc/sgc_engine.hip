@@ -202,6 +202,7 @@ struct BatchRun {
     sgc_batch_config cfg{};
     uint32_t rounds = 0, ng = 0, max_count = 0, sweeps = 0, ovf_cap = 0, t2_passes = 0;
     uint32_t sweeps_max = 0;                   // most Tier-1 sweeps a capture may hold
+    uint64_t max_vertices = 0;                 // of the graphs of the round with max_count records
     uint64_t updates = 0;
     bool multi = false, any_history = false, all_settled = true;
     bool lean = false;                         // captures leave the Tier-2 check and repair out
@@ -484,6 +485,11 @@ struct sgc_pool {
         return timed("build_list", [&] {
             return launch_build_list(L, kind, d_list, list_cap, d_list_count, later, second_list());
         });
+    }
+    uint64_t vertices(const std::vector<uint32_t>& gids) const {
+        uint64_t sum = 0;
+        for (uint32_t g : gids) sum += gs[g].n;
+        return sum;
     }
     size_t second_list() const { return list_words(list_cap, max_graphs); }
     // The sweep that follows an epoch's compaction and drain over the same
@@ -782,8 +788,10 @@ int sgc_pool::apply(const sgc_edge_update* upd, uint32_t count, bool on_device, 
         if (e == hipSuccess)
             e = timed("apply", [&] { return launch_apply_seg(L, src, seg.d, nseg, multi ? perm.d : nullptr, multi); });
     } else {
+        uint64_t verts = 0;
+        for (uint32_t g = 0; g < ng; g++) verts += per_graph[g] ? gs[g].n : 0u;
         e = timed("group", [&] { return launch_group(L, src, count, multi, &eg); });
-        if (e == hipSuccess) e = timed("apply", [&] { return launch_apply(L, src, count, multi, &eg); });
+        if (e == hipSuccess) e = timed("apply", [&] { return launch_apply(L, src, count, multi, &eg, verts); });
     }
     if (e != hipSuccess) return hip_fail(e, "apply launch");
     if (!on_device) {
@@ -1292,7 +1300,10 @@ int sgc_pool::batch_plan(const sgc_edge_update* upd, uint64_t count, const sgc_b
         }
         B->tab.push_back(off);
         B->tab.push_back((uint32_t)ordered.size() - off);
-        B->max_count = std::max(B->max_count, (uint32_t)ordered.size() - off);
+        if ((uint32_t)ordered.size() - off > B->max_count) {
+            B->max_count = (uint32_t)ordered.size() - off;
+            B->max_vertices = vertices(in);
+        }
         B->gids.push_back(in);
         B->rounds++;
     }
@@ -1432,7 +1443,8 @@ int sgc_pool::batch_capture(const sgc_tuning& t, hipGraphExec_t* out) {
             e = launch_apply_seg(La, B.d_stream, B.d_seg, ng, nullptr, B.multi ? 1 : 0);
         } else {
             e = launch_group(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg);
-            if (e == hipSuccess) e = launch_apply(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg);
+            if (e == hipSuccess)
+                e = launch_apply(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg, B.max_vertices);
         }
     }
     LaunchCtx Lr = base;
@@ -1615,7 +1627,9 @@ int sgc_pool::batch_run_host(BatchRun& B) {
         } else {
             e = timed("group", [&] { return launch_group(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg); });
             if (e == hipSuccess)
-                e = timed("apply", [&] { return launch_apply(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg); });
+                e = timed("apply", [&] {
+                    return launch_apply(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg, vertices(B.gids[r]));
+                });
         }
         if (e != hipSuccess) return hip_fail(e, "batch apply");
         for (uint32_t g : B.gids[r]) gs[g].since_epoch += B.counts[(size_t)r * ng + g];

@@ -515,6 +515,78 @@ __device__ __forceinline__ void apply_record(const GraphDev* __restrict__ graphs
     apply_rec(graphs, upd[i], multi, acc, hint);
 }
 
+__device__ __forceinline__ uint4 uniform_rec(const uint4& r) {
+    return make_uint4(bcast0(r.x), bcast0(r.y), bcast0(r.z), bcast0(r.w));
+}
+
+// Listed edge j's updates in stream order, by the whole wavefront.  The records
+// come from the edge's packed 64-byte line (lanes 0..3 load one each), or, for a
+// group longer than the line, from its list: repeatedly the record at the
+// smallest position above the last one applied.
+// SCALAR: the record in scalar registers.  Alone the update's code takes 165
+// vector registers and spills 34 scalar ones without it, 138 and 182 with it,
+// and 4,099 updates of a 65,536-vertex R-MAT graph take 45 us without and 48-64
+// with it.  Beside the four-edge path it is the other way round: without it the
+// kernel spills 64 vector registers into 52 B of scratch a lane, with it none.
+template <bool SCALAR>
+__device__ __forceinline__ void apply_edge(const GraphDev* __restrict__ graphs, const uint4* __restrict__ upd, int multi,
+                                           const uint32_t* __restrict__ gnext, const uint4* __restrict__ pack, uint32_t j,
+                                           WaveAcc& acc, uint64_t& grouped) {
+    uint4 mine = make_uint4(PACK_NONE, PACK_WALK, 0u, 0u);
+    if (lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
+    const bool walk = __builtin_amdgcn_readlane(mine.x, 0) == PACK_NONE &&
+                      __builtin_amdgcn_readlane(mine.y, 0) == PACK_WALK;
+    const uint32_t h = walk ? pack[(size_t)j * GROUP_PACK].w : NONE;   // the list's first position
+    RowHint hint;   // a delete's slots for the same edge's re-insert (a last delete's marks wait in it)
+    hint.valid = false;
+    uint32_t applied = 0, last = 0, last_g = 0;
+    for (;;) {
+        uint4 r;
+        if (!walk) {
+            if (applied == GROUP_PACK) break;
+            r = make_uint4(__builtin_amdgcn_readlane(mine.x, applied), __builtin_amdgcn_readlane(mine.y, applied),
+                           __builtin_amdgcn_readlane(mine.z, applied), __builtin_amdgcn_readlane(mine.w, applied));
+            if (r.x == PACK_NONE) break;
+        } else {
+            uint32_t best = NONE;
+            for (uint32_t k2 = h; k2 != NONE; k2 = gp(gnext)[k2])
+                if ((applied == 0 || k2 > last) && (best == NONE || k2 < best)) best = k2;
+            if (best == NONE) break;
+            r = upd[best];
+            last = best;
+        }
+        apply_rec(graphs, SCALAR ? uniform_rec(r) : r, multi, acc, &hint);
+        last_g = r.w;
+        applied++;
+    }
+    if (hint.valid) hint_release(graphs[multi ? last_g : 0u], &hint);   // marks of a last delete
+    grouped += applied ? applied - 1 : 0;
+}
+
+// One wavefront per edge of the batch.
+__global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ graphs, const uint4* __restrict__ upd,
+                                                   uint32_t count, int multi, const uint32_t* __restrict__ gnext,
+                                                   uint32_t* __restrict__ nheads, const uint4* __restrict__ pack,
+                                                   uint64_t* totals, const uint32_t* __restrict__ dyn) {
+    WaveAcc acc;
+    uint64_t grouped = 0;
+    if (dyn) {
+        upd += dyn[0];
+        count = dyn[1];
+    }
+    if (!pack) {   // no grouping: one wavefront per position
+        for (uint32_t i = wave_id(); i < count; i += wave_count()) apply_record(graphs, upd, i, multi, acc);
+        acc.flush(totals);
+        return;
+    }
+    const uint32_t n = nheads[2] + nheads[3];
+    if (blockIdx.x == 0 && lane() < 2) nheads[lane()] = 0;   // for the next batch's k_group_link
+    for (uint32_t j = wave_id(); j < n; j += wave_count())
+        apply_edge<false>(graphs, upd, multi, gnext, pack, j, acc, grouped);
+    acc.flush(totals);
+    if (grouped && totals && lane() == 0) tot_add(totals, T_GROUPED, grouped);
+}
+
 // ---- four light edges to a wavefront
 // An edge with short rows keeps a wavefront's lanes mostly idle, and the chip
 // runs out of wavefront slots long before it runs out of anything else: the
@@ -798,38 +870,20 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
     if (act && held_x != INVALID && lead) mark(g, held_x, held);   // marks of a last delete
 }
 
-// One wavefront per heavy edge of the batch, then one per four light ones.  Up
-// to APPLY_SPREAD light edges take a wavefront each: the chip runs some 3,000
-// wavefronts of this kernel (3 a SIMD, for its 168 registers) and one edge's
-// chain is shorter alone (1,338 light edges of a 65,536-vertex R-MAT graph,
-// launch: 37 us alone, 45 us by fours).  Launch times with one edge a wavefront
-// and scans of 512 slots a trip / now: 32,768 updates of a 131,072-vertex mesh
-// 56 / 38 us, of the 4M-vertex power-law graph 100 / 71, of dense growth on a
-// 2^18-vertex R-MAT graph 157 / 131; 4,099 updates of the 65,536-vertex one
-// 56 / 44; a pool's 262K updates 308 / 191.  Bound: the chain of dependent
-// gathers and atomics of an edge, over the wavefronts the registers allow.
+// One wavefront per heavy edge of the batch, then one per four light ones (if
+// they are enough to fill the chip, some 3,000 wavefronts of this kernel).
+// Bound: the chain of dependent gathers and atomics of an edge, over the
+// wavefronts the registers allow.
 constexpr uint32_t APPLY_SPREAD = 4096;
-__global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict__ graphs,
-                                                    const uint4* __restrict__ upd, uint32_t count, int multi,
-                                                    const uint32_t* __restrict__ gnext,
-                                                    uint32_t* __restrict__ nheads,
-                                                    const uint4* __restrict__ pack, uint64_t* totals,
-                                                    const uint32_t* __restrict__ dyn) {
+__global__ __launch_bounds__(64, 3) void k_apply_quads(const GraphDev* __restrict__ graphs,
+                                                       const uint4* __restrict__ upd, int multi,
+                                                       const uint32_t* __restrict__ gnext,
+                                                       uint32_t* __restrict__ nheads,
+                                                       const uint4* __restrict__ pack, uint64_t* totals,
+                                                       const uint32_t* __restrict__ dyn) {
     WaveAcc acc;
     uint64_t grouped = 0;
-    if (dyn) {
-        upd += dyn[0];
-        count = dyn[1];
-    }
-    if (!pack) {   // no grouping: one wavefront per position
-        for (uint32_t i = wave_id(); i < count; i += wave_count()) apply_record(graphs, upd, i, multi, acc);
-        acc.flush(totals);
-        return;
-    }
-    // An edge's updates in stream order.  The records come from the edge's
-    // packed 64-byte line (one lane each), or, for a group longer than the
-    // line, from its list: repeatedly the record at the smallest position
-    // above the last one applied.
+    if (dyn) upd += dyn[0];
     const uint32_t nh = nheads[2], nl = nheads[3];
     if (blockIdx.x == 0 && lane() < 2) nheads[lane()] = 0;   // for the next batch's k_group_link
     const uint32_t per = nl > APPLY_SPREAD ? GROUPS : 1u;
@@ -860,40 +914,8 @@ __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict
             const uint64_t left = ballot(have && !quad && sublane() == 0);
             for (uint32_t i = 0; i < GROUPS; i++) whole |= (uint32_t)((left >> (GROUP * i)) & 1u) << i;
         }
-        for (; whole; whole &= whole - 1) {
-            const uint32_t j = j0 + (uint32_t)__builtin_ctz(whole);
-            uint4 mine = make_uint4(PACK_NONE, PACK_WALK, 0u, 0u);
-            if (lane() < GROUP_PACK) mine = pack[(size_t)j * GROUP_PACK + lane()];
-            const bool walk = __builtin_amdgcn_readlane(mine.x, 0) == PACK_NONE &&
-                              __builtin_amdgcn_readlane(mine.y, 0) == PACK_WALK;
-            const uint32_t h = __builtin_amdgcn_readlane(mine.w, 0);   // the list's first position
-            RowHint hint;   // a delete's slots for the same edge's re-insert (a last delete's marks wait in it)
-            hint.valid = false;
-            uint32_t applied = 0, last = 0, last_g = 0;
-            for (;;) {
-                uint4 r;
-                if (!walk) {
-                    if (applied == GROUP_PACK) break;
-                    r = make_uint4(__builtin_amdgcn_readlane(mine.x, applied),
-                                   __builtin_amdgcn_readlane(mine.y, applied),
-                                   __builtin_amdgcn_readlane(mine.z, applied),
-                                   __builtin_amdgcn_readlane(mine.w, applied));
-                    if (r.x == PACK_NONE) break;
-                } else {
-                    uint32_t best = NONE;
-                    for (uint32_t k2 = h; k2 != NONE; k2 = gp(gnext)[k2])
-                        if ((applied == 0 || k2 > last) && (best == NONE || k2 < best)) best = k2;
-                    if (best == NONE) break;
-                    r = upd[best];
-                    last = best;
-                }
-                apply_rec(graphs, r, multi, acc, &hint);
-                last_g = r.w;
-                applied++;
-            }
-            if (hint.valid) hint_release(graphs[multi ? last_g : 0u], &hint);   // marks of a last delete
-            grouped += applied ? applied - 1 : 0;
-        }
+        for (; whole; whole &= whole - 1)
+            apply_edge<true>(graphs, upd, multi, gnext, pack, j0 + (uint32_t)__builtin_ctz(whole), acc, grouped);
     }
     if (per > 1) {
         acc.updates += wave_sum32(lanes.updates);
@@ -904,10 +926,6 @@ __global__ __launch_bounds__(64, 3) void k_apply_elem(const GraphDev* __restrict
     }
     acc.flush(totals);
     if (grouped && totals && lane() == 0) tot_add(totals, T_GROUPED, grouped);
-}
-
-__device__ __forceinline__ uint4 uniform_rec(const uint4& r) {
-    return make_uint4(bcast0(r.x), bcast0(r.y), bcast0(r.z), bcast0(r.w));
 }
 
 // One block per segment, the segment's updates in stream order (deterministic
@@ -2550,16 +2568,34 @@ static inline uint32_t grid_for_waves(uint64_t waves, uint32_t waves_per_block, 
     return (uint32_t)b;
 }
 
-hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg) {
+// Four light edges to a wavefront for more than QUADS_OVER updates: below, the
+// chip holds most of the edges at once, one to a wavefront, and an edge's chain
+// is shorter alone (launch, us, one / four edges a wavefront: 5,400 updates of a
+// 131,072-vertex mesh 16.5 / 18, 8,193: 22.5 / 15; 4,099 of a 65,536-vertex
+// R-MAT graph 45 / 52, 8,193: 81 / 81).  And for at most one update to two
+// vertices: with more, updates meet at the same rows, all the more of them the
+// more are in flight, and an edge's colour choices wait for three others'
+// (16,384 updates of growth on an 8,192-vertex R-MAT graph 118 / 207, 32,768 of
+// churn on a 16,384-vertex one 150 / 220; at one to two, 65,536 updates: a
+// 131,072-vertex mesh 107 / 58, an R-MAT graph of that size 285 / 269, of growth
+// 281 / 231, but 16,384 on a 32,768-vertex one 106 / 111; 196,608 of 48 graphs,
+// one to 2.4, 331 / 194).
+constexpr uint32_t QUADS_OVER = 8192;
+hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg,
+                        uint64_t vertices) {
     if (count == 0) return hipSuccess;
     const bool group = eg && eg->keys && count > 1;
     if (group && ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->heads || !eg->nheads || !eg->pack))
         return hipErrorInvalidValue;
     const EdgeGroups G = group ? *eg : EdgeGroups();
     // one-wavefront blocks: a wavefront's slot is refilled as soon as it ends
-    uint32_t grid = grid_for_waves(count, 1, 4 * L.max_blocks);
-    k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, G.next, G.nheads, G.pack,
-                                               L.totals, L.dyn);
+    const uint32_t grid = grid_for_waves(count, 1, 4 * L.max_blocks);
+    if (group && count > QUADS_OVER && count <= vertices / 2)
+        k_apply_quads<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
+                                                   L.totals, L.dyn);
+    else
+        k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, G.next, G.nheads, G.pack,
+                                                  L.totals, L.dyn);
     return hipGetLastError();
 }
 hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg) {

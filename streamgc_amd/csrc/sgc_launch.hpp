@@ -59,7 +59,9 @@ constexpr uint32_t GROUP_WORDS = 4;
 hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg);
 // Per-edge grouping of a parallel batch (before launch_apply with the same eg).
 hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg);
-hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg);
+// vertices: of the graphs that the batch updates.
+hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg,
+                        uint64_t vertices);
 hipError_t launch_apply_seg(const LaunchCtx& L, const void* upd, const uint32_t* seg, uint32_t nseg,
                             const uint32_t* perm, int multi);
 hipError_t launch_zero_ctr(const LaunchCtx& L, uint32_t idx);

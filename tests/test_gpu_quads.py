@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import streamgc_amd as S
+import test_gpu_apply
 from test_gpu_parity import _pair
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,32 @@ def test_deletes_and_inserts_at_one_vertex(threshold):
     assert np.array_equal(_rows(gpu.csr()), _rows(orc.csr()))
     assert np.array_equal(gpu.hist(), orc.hist())
     assert np.all(orc.bitmaps() & ~gpu.bitmaps() == 0)   # (no neighbour's colour is missing)
+
+
+@pytest.mark.parametrize("slack,cap", [(300, 0), (0, 1), (50, 2)])
+@pytest.mark.parametrize("graphs", [1, 3])
+def test_light_edges_by_four(graphs, slack, cap, monkeypatch):
+    """The disjoint light edges of test_gpu_apply, more of them and over twice as many vertices as updates."""
+    plain = test_gpu_apply._light_graph
+
+    def sparse():
+        g = plain()
+        return S.CSRGraph(g.n + 12000, np.concatenate([g.row_ptr, np.full(12000, g.row_ptr[-1])]), g.col_idx)
+    monkeypatch.setattr(test_gpu_apply, "PAIRS", 6500)
+    monkeypatch.setattr(test_gpu_apply, "_light_graph", sparse)
+    test_gpu_apply.test_light_edges_keep_the_oracles_slots(graphs, slack, cap)
+
+
+@pytest.mark.parametrize("pairs", [4097, 8192, 8193, 8196, 9217])
+def test_where_light_edges_go_by_four(pairs):
+    """Launches at and past the least number of updates, and with one to two vertices and one more."""
+    g = S.csr_from_edges(2 * pairs, [(2 * i, 2 * i + 1) for i in range(pairs)])
+    gpu, orc, og = _pair(g, epoch_size=1 << 20, batch_size=1 << 20)
+    u = 2 * np.arange(pairs, dtype=np.uint32)
+    for extra, kind in ((0, 1), (1, 0), (0, 1)):
+        recs = S.make_updates(np.concatenate([u, u[:extra]]), np.concatenate([u + 1, u[:extra] + 1]),
+                              np.full(pairs + extra, kind, np.uint8))
+        gpu.apply(recs)
+        orc.submit(recs["u"], recs["v"], recs["type"])
+        assert np.array_equal(gpu.csr()[1], orc.csr()[1]), (pairs, extra)
+        assert np.array_equal(gpu.words() & 0xFFFF, orc.words() & 0xFFFF), (pairs, extra)
