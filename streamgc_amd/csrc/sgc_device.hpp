@@ -34,12 +34,9 @@ constexpr uint32_t ROW_UNROLL = 4;
 // other is done: a hub row's search takes SCAN_CHUNKS x 64 slots per trip.
 // 8 rather than 16: every trip runs the code of all SCAN_CHUNKS chunks, and
 // the shorter trips made the per-update kernel 8% faster on a 4M-vertex
-// power-law graph although hub rows take twice as many of them.  Trips of
-// 1,024 slots by another loop make a hub's deletes twice as fast (a 37.5K-slot
-// row 90 -> 41 us), but updates of one launch that meet at a vertex are settled
-// by the order in which they get there: with them, 3 of 65,536 vertices of a
-// skewed graph's churn ended with another colour, and a graph coloured from its
-// edges took 84-87 colours instead of 81-83.
+// power-law graph although hub rows take twice as many of them.
+// While more than that is left of a row, long_search takes over in launches that
+// scan so (LONG).
 constexpr uint32_t SCAN_CHUNKS = 8;
 constexpr int MAX_CAS_RETRIES = 64;          // recolour CAS retries before leaving it to repair
 // Ablation flags carried by the descriptors (the values of SGC_ABL_* in streamgc.h).
@@ -138,6 +135,13 @@ __device__ __forceinline__ uint64_t wave_min64(uint64_t x) {
 }
 __device__ __forceinline__ uint32_t wave_sum32(uint32_t x) {
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_min32(uint32_t x) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t y = __shfl_xor(x, o);
+        x = y < x ? y : x;
+    }
     return x;
 }
 __device__ __forceinline__ uint32_t wave_max32(uint32_t x) {
@@ -324,6 +328,54 @@ __device__ __forceinline__ void on_neighbor_recolor(const GraphDev& g, uint32_t 
 }
 
 // ---------------------------------------------------------------- slack-CSR rows
+// The first slot of [b, end) that holds `want`, or INVALID.  free: the first
+// free slot passed, if none was before.  For rows with more than LONG_SCAN
+// slots to go: one trip loads 8 pairs of slots a lane, 1,024 slots, where a
+// trip of scan_pair takes 512.  A hub row's scan is one chain of such trips
+// (1.2-1.5 us each), and the longest chain ends the launch: of 32,768 updates
+// of the 4M-vertex power-law graph one read 37.5K slots in 90 of the launch's
+// 91 us, so in 41.  16 pairs take 215 registers in the per-update kernel, which
+// leaves it 2 wavefronts a SIMD instead of 3.
+constexpr uint32_t LONG_SCAN = SCAN_CHUNKS * WAVE;
+__device__ __forceinline__ uint32_t long_search(const GraphDev& g, uint32_t b, uint32_t end, uint32_t want,
+                                                uint32_t& free) {
+    constexpr uint32_t PAIRS = 8, STEP = 2 * WAVE;
+    const uint64_t none = want ? 0ull : 1ull | 1ull << 32;   // neither want nor free
+    const auto first_of = [](uint32_t m, uint32_t j) {       // the wave's first slot of the lanes' masks
+        uint32_t at = INVALID;
+        if (m) {
+            const uint32_t k = (uint32_t)__builtin_ctz(m);
+            at = j + (k >> 1) * STEP + (k & 1u);
+        }
+        return wave_min32(at);
+    };
+    // pairs start at even slots (the slot array is padded to a whole pair)
+    for (uint32_t a = b & ~1u; a < end; a += PAIRS * STEP) {
+        const uint32_t j = a + 2 * lane(), left = end > j ? end - j : 0u;
+        uint64_t p[PAIRS];
+#pragma unroll
+        for (uint32_t q = 0; q < PAIRS; q++)
+            p[q] = q * STEP < left ? ld((const uint64_t*)(g.col + j + q * STEP)) : none;
+        uint32_t ok = j < b ? ~1u : ~0u;   // a slot before b, a slot past the end
+        if (left % STEP == 1 && left / STEP < PAIRS) ok &= ~(2u << (2 * (left / STEP)));
+        uint32_t hit = 0, hole = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < PAIRS; q++)
+            hit |= (uint32_t)((uint32_t)p[q] == want) << (2 * q) | (uint32_t)((uint32_t)(p[q] >> 32) == want) << (2 * q + 1);
+        hit &= ok;
+        if (free == INVALID) {
+#pragma unroll
+            for (uint32_t q = 0; q < PAIRS; q++)
+                hole |= (uint32_t)((uint32_t)p[q] == INVALID) << (2 * q) |
+                        (uint32_t)((uint32_t)(p[q] >> 32) == INVALID) << (2 * q + 1);
+            hole &= ok;
+            if (ballot(hole != 0)) free = first_of(hole, j);
+        }
+        if (ballot(hit != 0)) return first_of(hit, j);
+    }
+    return INVALID;
+}
+
 // An insert that lands in a hole may duplicate a copy further along the row
 // (the first-free-or-equal scan meets the hole first,
 // A/src/kernels/local_update.cu:12-40); a later delete then removes one copy
@@ -453,7 +505,13 @@ __device__ __forceinline__ void mark_neighbors(const GraphDev& g, uint32_t v, ui
 // pf = the fill before an insert's raise when this wave wrote the slot, else 0;
 // had = an insert found the neighbour in the row already; free = the first
 // free slot a delete's scan passed (absolute index, INVALID: none).
-template <bool INSERT>
+// LONG: a delete's rows with more than LONG_SCAN slots to go are scanned by
+// long_search.  Inserts keep to the short trips: a hub's inserts then come to
+// their colour choices one after another, as far as their edges lie in its row.
+// All at once they cost colours (the 4M-vertex power-law graph coloured from
+// its edges in launches of 256: 84-87 colours in 6 runs, 81-83 in 8 with the
+// short trips; the sequential replay has 83).
+template <bool INSERT, bool LONG>
 __device__ __forceinline__ void scan_pair(const GraphDev& g, bool run0, uint32_t x0, uint32_t nb0, uint32_t s0,
                                           uint32_t end0, bool run1, uint32_t x1, uint32_t nb1, uint32_t s1,
                                           uint32_t end1, uint32_t& pos0, uint32_t& pos1, uint32_t& pf0,
@@ -508,24 +566,39 @@ __device__ __forceinline__ void scan_pair(const GraphDev& g, bool run0, uint32_t
     while (run0 || run1) {
         c0 = c1 = INVALID;
         eq0 = eq1 = false;
-        uint32_t per0, per1;
-        if (run0 && run1 && end0 - b0 <= WAVE && end1 - b1 <= WAVE) {
-            // Both rows end within one chunk: a trip of two chunks (light
-            // rows, the common case, run far fewer instructions).
-            per0 = per1 = 1;
-            trip(std::integral_constant<uint32_t, 2>{}, per0, per1);
+        const bool long0 = !INSERT && LONG && run0 && end0 - b0 > LONG_SCAN;
+        const bool long1 = !INSERT && LONG && run1 && end1 - b1 > LONG_SCAN;
+        if (long0 || long1) {
+            // one row of the two (one copy of the code), the other at the next turn
+            uint32_t fr = long0 ? free0 : free1;
+            const uint32_t at = long_search(g, long0 ? b0 : b1, long0 ? end0 : end1, long0 ? nb0 : nb1, fr);
+            if (long0) {
+                c0 = at, free0 = fr;
+                run0 = at != INVALID;
+            } else {
+                c1 = at, free1 = fr;
+                run1 = at != INVALID;
+            }
         } else {
-            per0 = run0 ? (run1 ? ROW_UNROLL : CH) : 0;
-            per1 = run1 ? (run0 ? ROW_UNROLL : CH) : 0;
-            trip(std::integral_constant<uint32_t, CH>{}, per0, per1);
-        }
-        if (run0 && c0 == INVALID) {
-            b0 += per0 * WAVE;
-            run0 = b0 < end0;
-        }
-        if (run1 && c1 == INVALID) {
-            b1 += per1 * WAVE;
-            run1 = b1 < end1;
+            uint32_t per0, per1;
+            if (run0 && run1 && end0 - b0 <= WAVE && end1 - b1 <= WAVE) {
+                // Both rows end within one chunk: a trip of two chunks (light
+                // rows, the common case, run far fewer instructions).
+                per0 = per1 = 1;
+                trip(std::integral_constant<uint32_t, 2>{}, per0, per1);
+            } else {
+                per0 = run0 ? (run1 ? ROW_UNROLL : CH) : 0;
+                per1 = run1 ? (run0 ? ROW_UNROLL : CH) : 0;
+                trip(std::integral_constant<uint32_t, CH>{}, per0, per1);
+            }
+            if (run0 && c0 == INVALID) {
+                b0 += per0 * WAVE;
+                run0 = b0 < end0;
+            }
+            if (run1 && c1 == INVALID) {
+                b1 += per1 * WAVE;
+                run1 = b1 < end1;
+            }
         }
         if (INSERT && c0 != INVALID && eq0) {   // the neighbour is there already
             pos0 = c0 - s0 + 1;
@@ -759,6 +832,7 @@ __device__ __forceinline__ void hint_release(const GraphDev& g, RowHint* h) {
     }
     h->valid = false;
 }
+template <bool LONG>
 __device__ __forceinline__ void apply_update(const GraphDev& g, uint32_t u, uint32_t v, uint32_t type, WaveAcc& acc,
                                              RowHint* hint = nullptr) {
     const bool hinted = type == 0 && hint && hint->valid && hint->u == u && hint->v == v && u < g.n && v < g.n;
@@ -813,10 +887,10 @@ __device__ __forceinline__ void apply_update(const GraphDev& g, uint32_t u, uint
         if (scan_u || scan_v) {
             uint32_t qu, qv, gu, gv;
             bool au, av;
-            scan_pair<true>(g, scan_u, u, v, su, eu, two && scan_v, v, u, sv, ev, qu, qv, gu, gv, au, av, xu, xv);
+            scan_pair<true, false>(g, scan_u, u, v, su, eu, two && scan_v, v, u, sv, ev, qu, qv, gu, gv, au, av, xu, xv);
             if (scan_u) pu = qu, fu = gu, hadu = au;
             if (scan_v && two) pv = qv, fv = gv, hadv = av;
-            if (!two) scan_pair<true>(g, false, u, v, su, eu, true, v, u, sv, ev, d0, pv, d1, fv, h0, hadv, xu, xv);
+            if (!two) scan_pair<true, false>(g, false, u, v, su, eu, true, v, u, sv, ev, d0, pv, d1, fv, h0, hadv, xu, xv);
         }
         // No duplicate check when both rows took the slots the delete left:
         // each row lost one copy of the edge and gained one, so the rows hold
@@ -864,8 +938,8 @@ __device__ __forceinline__ void apply_update(const GraphDev& g, uint32_t u, uint
         const uint64_t bu = ld(&g.bitmap[u]), bv = ld(&g.bitmap[v]);   // for the reductions below
         const uint16_t cu = color_of(bcast0(ru)), cv = color_of(bcast0(rv));   // freed at v, freed at u
         const uint32_t tu = su + bcast0(lu), tv = sv + bcast0(lv);
-        scan_pair<false>(g, true, u, v, su, tu, two, v, u, sv, tv, pu, pv, fu, fv, hadu, hadv, xu, xv);
-        if (!two) scan_pair<false>(g, false, u, v, su, tu, true, v, u, sv, tv, d0, pv, d1, fv, h0, hadv, d0, xv);
+        scan_pair<false, LONG>(g, true, u, v, su, tu, two, v, u, sv, tv, pu, pv, fu, fv, hadu, hadv, xu, xv);
+        if (!two) scan_pair<false, LONG>(g, false, u, v, su, tu, true, v, u, sv, tv, d0, pv, d1, fv, h0, hadv, d0, xv);
         acc.scan += (pu ? pu : tu - su) + (pv ? pv : tv - sv);
         const uint32_t mu = (pu ? D_ROW : 0u) | ((hu == INVALID) == (pu != 0) ? D_BITS : 0u);
         const uint32_t mv = (pv ? D_ROW : 0u) | ((hv == INVALID) == (pv != 0) ? D_BITS : 0u);

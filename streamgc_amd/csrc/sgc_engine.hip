@@ -627,7 +627,7 @@ int sgc_pool::add_graph(const sgc_config* cfg, uint32_t n, const uint32_t* row_p
     A((void**)&G.word, (size_t)n * 4);
     A((void**)&G.deg0, (size_t)n * 4);
     A((void**)&G.row_ptr, ((size_t)n + 1) * 4);
-    A((void**)&G.col, (S + (S & 1)) * 4);   // light edges' scans read whole pairs of slots
+    A((void**)&G.col, (S + (S & 1)) * 4);   // light edges' scans and long ones read whole pairs of slots
     A((void**)&G.fill, (size_t)mark_stride(n) * 4);   // padded: sweeps read fill 4 vertices at a time
     A((void**)&G.bitmap, (size_t)n * 8);
     A((void**)&G.hd_map, (size_t)n * 4);

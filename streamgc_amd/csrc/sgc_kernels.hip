@@ -504,11 +504,12 @@ __global__ __launch_bounds__(256) void k_group_pack(const uint4* __restrict__ up
 }
 
 // ---------------------------------------------------------------- updates
+template <bool LONG = false>
 __device__ __forceinline__ void apply_rec(const GraphDev* __restrict__ graphs, const uint4& r, int multi, WaveAcc& acc,
                                           RowHint* hint = nullptr) {
     const uint32_t gid = multi ? r.w : 0u;
     const GraphDev g = graphs[gid];
-    apply_update(g, r.x, r.y, r.z & 0xFFu, acc, hint);
+    apply_update<LONG>(g, r.x, r.y, r.z & 0xFFu, acc, hint);
 }
 __device__ __forceinline__ void apply_record(const GraphDev* __restrict__ graphs, const uint4* __restrict__ upd,
                                              uint32_t i, int multi, WaveAcc& acc, RowHint* hint = nullptr) {
@@ -528,7 +529,7 @@ __device__ __forceinline__ uint4 uniform_rec(const uint4& r) {
 // and 4,099 updates of a 65,536-vertex R-MAT graph take 45 us without and 48-64
 // with it.  Beside the four-edge path it is the other way round: without it the
 // kernel spills 64 vector registers into 52 B of scratch a lane, with it none.
-template <bool SCALAR>
+template <bool SCALAR, bool LONG>
 __device__ __forceinline__ void apply_edge(const GraphDev* __restrict__ graphs, const uint4* __restrict__ upd, int multi,
                                            const uint32_t* __restrict__ gnext, const uint4* __restrict__ pack, uint32_t j,
                                            WaveAcc& acc, uint64_t& grouped) {
@@ -555,7 +556,7 @@ __device__ __forceinline__ void apply_edge(const GraphDev* __restrict__ graphs, 
             r = upd[best];
             last = best;
         }
-        apply_rec(graphs, SCALAR ? uniform_rec(r) : r, multi, acc, &hint);
+        apply_rec<LONG>(graphs, SCALAR ? uniform_rec(r) : r, multi, acc, &hint);
         last_g = r.w;
         applied++;
     }
@@ -582,7 +583,7 @@ __global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ 
     const uint32_t n = nheads[2] + nheads[3];
     if (blockIdx.x == 0 && lane() < 2) nheads[lane()] = 0;   // for the next batch's k_group_link
     for (uint32_t j = wave_id(); j < n; j += wave_count())
-        apply_edge<false>(graphs, upd, multi, gnext, pack, j, acc, grouped);
+        apply_edge<false, false>(graphs, upd, multi, gnext, pack, j, acc, grouped);
     acc.flush(totals);
     if (grouped && totals && lane() == 0) tot_add(totals, T_GROUPED, grouped);
 }
@@ -875,6 +876,7 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
 // Bound: the chain of dependent gathers and atomics of an edge, over the
 // wavefronts the registers allow.
 constexpr uint32_t APPLY_SPREAD = 4096;
+template <bool LONG>
 __global__ __launch_bounds__(64, 3) void k_apply_quads(const GraphDev* __restrict__ graphs,
                                                        const uint4* __restrict__ upd, int multi,
                                                        const uint32_t* __restrict__ gnext,
@@ -915,7 +917,7 @@ __global__ __launch_bounds__(64, 3) void k_apply_quads(const GraphDev* __restric
             for (uint32_t i = 0; i < GROUPS; i++) whole |= (uint32_t)((left >> (GROUP * i)) & 1u) << i;
         }
         for (; whole; whole &= whole - 1)
-            apply_edge<true>(graphs, upd, multi, gnext, pack, j0 + (uint32_t)__builtin_ctz(whole), acc, grouped);
+            apply_edge<true, LONG>(graphs, upd, multi, gnext, pack, j0 + (uint32_t)__builtin_ctz(whole), acc, grouped);
     }
     if (per > 1) {
         acc.updates += wave_sum32(lanes.updates);
@@ -2581,6 +2583,17 @@ static inline uint32_t grid_for_waves(uint64_t waves, uint32_t waves_per_block, 
 // 281 / 231, but 16,384 on a 32,768-vertex one 106 / 111; 196,608 of 48 graphs,
 // one to 2.4, 331 / 194).
 constexpr uint32_t QUADS_OVER = 8192;
+// A delete's long scans in trips of 1,024 slots for at most one update to
+// LONG_PER vertices.  They end a hub's deletes in half the time, and so before
+// other updates of the launch that touch the same vertices: on a skewed graph
+// with one update to 16 vertices some streams then end with other colours every
+// time (tests/test_gpu_racing.py).  At one to 64 and fewer, updates hardly meet:
+// of 108 passes of such streams on five graphs 106 ended as the short trips' did,
+// as many as between two runs of the short trips.  Launch, us, short / long trips: 32,768 updates
+// of a 4M-vertex power-law graph 125 / 78, 16,384 of a 2^20-vertex R-MAT graph
+// 325 / 197, of growth there 208 / 148; at one to 32, 16,384 of growth on a
+// 2^19-vertex one 142 / 152.
+constexpr uint32_t LONG_PER = 64;
 hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg,
                         uint64_t vertices) {
     if (count == 0) return hipSuccess;
@@ -2590,9 +2603,12 @@ hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int
     const EdgeGroups G = group ? *eg : EdgeGroups();
     // one-wavefront blocks: a wavefront's slot is refilled as soon as it ends
     const uint32_t grid = grid_for_waves(count, 1, 4 * L.max_blocks);
-    if (group && count > QUADS_OVER && count <= vertices / 2)
-        k_apply_quads<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
-                                                   L.totals, L.dyn);
+    if (group && count > QUADS_OVER && count <= vertices / LONG_PER)
+        k_apply_quads<true><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
+                                                         L.totals, L.dyn);
+    else if (group && count > QUADS_OVER && count <= vertices / 2)
+        k_apply_quads<false><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
+                                                          L.totals, L.dyn);
     else
         k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, G.next, G.nheads, G.pack,
                                                   L.totals, L.dyn);

@@ -95,3 +95,32 @@ def test_where_light_edges_go_by_four(pairs):
         orc.submit(recs["u"], recs["v"], recs["type"])
         assert np.array_equal(gpu.csr()[1], orc.csr()[1]), (pairs, extra)
         assert np.array_equal(gpu.words() & 0xFFFF, orc.words() & 0xFFFF), (pairs, extra)
+
+
+def test_long_rows_in_sparse_launches():
+    """Long rows' searches in launches of few updates for the graph's size, among light edges that go by four."""
+    bed, pairs = 4000, 8200
+    rng = np.random.default_rng(8)
+    edges = [(bed + k, int(x)) for k, d in enumerate(test_gpu_apply.LONG) for x in rng.choice(bed, size=d, replace=False)]
+    first = bed + len(test_gpu_apply.LONG)
+    edges += [(first + 2 * i, first + 2 * i + 1) for i in range(pairs)]
+    g = S.csr_from_edges(64 * (pairs + 100), edges)
+    gpu, orc, og = _pair(g, epoch_size=1 << 20, batch_size=1 << 20, slack_pct=3)
+    u = first + 2 * np.arange(pairs, dtype=np.uint32)
+    live = test_gpu_apply._live
+    for k in range(6):   # one update of each long row a launch: deletes, a re-insert, inserts, a delete
+        rows, used, recs = orc.csr(), set(), []
+        for x in range(bed, first):
+            row = [w for w in live(rows, x) if w not in used]
+            out = [w for w in range(bed) if w not in used and w not in set(row)]
+            w = row[(0, len(row) // 2, len(row) - 1)[(x + k) % 3]]
+            recs.append([(x, w, 1), (w, x, 1), (x, out[x % 5], 0), (x, w, 0), (out[0], x, 0), (x, w, 1)][k])
+            used |= {recs[-1][0], recs[-1][1]}
+        a, b, t = (np.array(c) for c in zip(*recs))
+        batch = S.make_updates(np.concatenate([a, u]), np.concatenate([b, u + 1]),
+                               np.concatenate([t, np.full(pairs, 1 - k % 2)]).astype(np.uint8))
+        gpu.apply(batch)
+        orc.submit(batch["u"], batch["v"], batch["type"])
+        got, want = gpu.csr()[1], orc.csr()[1]
+        assert np.array_equal(got, want), (k, np.nonzero(got != want)[0][:8])
+    assert gpu.overflow_count() == orc.overflow_count()
