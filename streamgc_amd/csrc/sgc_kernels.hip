@@ -935,7 +935,7 @@ __global__ __launch_bounds__(64, 3) void k_apply_quads(const GraphDev* __restric
 // mixed batch).  One wavefront replaying a segment spends its time on one
 // update's chain of dependent loads at a time (2.6 us an update, whatever the
 // graph's size), so the block's WAVES wavefronts take the next WAVES updates
-// and judge each at once, reading only (replay_plain): an update is plain if it
+// and judge each at once, reading only (replay_judge): an update is plain if it
 // changes no word and finds room in both rows, whatever the plain updates
 // before it in the window do.  Plain updates touch nothing but their own
 // endpoints' rows, fills, bitmaps, histograms and marks, so those before the
@@ -2629,22 +2629,27 @@ hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int
                                            eg->nheads, eg->pack, L.dyn);
     return hipGetLastError();
 }
-// Up to so many segments a block of wavefronts replays each, above it one
-// wavefront: with more segments than that the chip's wavefront slots are better
-// filled by one a segment (64 churn updates on each of n 200-vertex meshes, us
-// by blocks / by single wavefronts: 256: 50 / 155, 1024: 188 / 190, 2048:
-// 372 / 230; a stream that colours fresh vertices breaks even near 500).
-constexpr uint32_t REPLAY_MANY = 512;
+// A CU holds 20 wavefronts of this kernel: one block of REPLAY_WAVES, or two of
+// half as many.  Up to REPLAY_BLOCKS segments (one to a CU) take whole blocks, up
+// to twice as many half ones, above it one wavefront each: a segment that had to
+// wait for another's block would take twice as long, which a stream with nothing
+// to run together (it colours fresh vertices) does not make good.  300 updates on
+// each of n 4,096-vertex meshes, us, single wavefronts / whole blocks / half
+// blocks: churn, n = 256: 797 / 186 / -, 512: 941 / 380 / 344; first colourings,
+// 256: 1,384 / 1,388 / -, 512: 1,652 / 2,801 / 1,649.
+constexpr uint32_t REPLAY_BLOCKS = 256;
 hipError_t launch_apply_seg(const LaunchCtx& L, const void* upd, const uint32_t* seg, uint32_t nseg,
                             const uint32_t* perm, int multi) {
     if (nseg == 0) return hipSuccess;
     const uint32_t grid = grid_for_waves(nseg, 1, L.max_blocks);
-    if (nseg <= REPLAY_MANY)
-        k_apply_seg<REPLAY_WAVES><<<grid, REPLAY_WAVES * WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg,
-                                                                              perm, multi, L.totals, L.dyn);
-    else
-        k_apply_seg<1><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg, perm, multi, L.totals,
-                                                    L.dyn);
+    const auto replay = [&](auto waves) {
+        constexpr uint32_t W = decltype(waves)::value;
+        k_apply_seg<W><<<grid, W * WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, seg, nseg, perm, multi, L.totals,
+                                                        L.dyn);
+    };
+    if (nseg <= REPLAY_BLOCKS) replay(std::integral_constant<uint32_t, REPLAY_WAVES>{});
+    else if (nseg <= 2 * REPLAY_BLOCKS) replay(std::integral_constant<uint32_t, REPLAY_WAVES / 2>{});
+    else replay(std::integral_constant<uint32_t, 1>{});
     return hipGetLastError();
 }
 hipError_t launch_zero_ctr(const LaunchCtx& L, uint32_t idx) {
