@@ -99,6 +99,15 @@ __device__ __forceinline__ void for_rows(const GraphDev* __restrict__ graphs, co
         }
     }
 }
+// Every row, a wavefront each: f(g, gid, v).
+template <class F>
+__device__ __forceinline__ void for_each_row(const GraphDev* __restrict__ graphs, const Space& sp, F&& f) {
+    for (uint32_t k = wave_id(); k < sp.total; k += wave_count()) {
+        uint32_t gid, v;
+        sp.locate(k, gid, v);
+        f(graphs[gid], gid, v);
+    }
+}
 // The rows of `m` (a lane mask), one after another by the whole wavefront: f(v).
 template <class F>
 __device__ __forceinline__ void each_row(uint64_t m, uint32_t v, F&& f) {
@@ -1381,6 +1390,8 @@ __device__ __forceinline__ void drain_prep_graph(const GraphDev* __restrict__ gr
 // prep_ng > 0: block 0 also takes the drain's counter snapshot of the
 // active graphs (k_drain_prep), which the drain launched next reads;
 // compaction touches none of those counters.
+// ALONE: a full sweep on a grid with a wavefront for every row (alone_rows).
+template <bool ALONE>
 __global__ __launch_bounds__(256, 8) void k_compact(const GraphDev* __restrict__ graphs, Space sp, SweepList sl,
                                                  uint64_t* totals, uint32_t prep_ng,
                                                  const uint32_t* __restrict__ prep_active) {
@@ -1388,6 +1399,18 @@ __global__ __launch_bounds__(256, 8) void k_compact(const GraphDev* __restrict__
         for (uint32_t gid = threadIdx.x; gid < prep_ng; gid += blockDim.x)
             if (!prep_active || prep_active[gid]) drain_prep_graph(graphs, gid);
     uint64_t live_total = 0, rows = 0, slots = 0;
+    if (ALONE) {
+        for_each_row(graphs, sp, [&](const GraphDev& g, uint32_t, uint32_t v) {
+            slots += gp(g.fill)[v];
+            live_total += compact_row_wave(g, v);
+            rows++;
+        });
+        if (lane() != 0) live_total = rows = slots = 0;
+        block_add64(totals, T_LIVE_SLOTS, live_total);
+        block_add64(totals, T_SWEEP_ROWS + 0, rows);
+        block_add64(totals, T_SWEEP_SLOTS + 0, slots);
+        return;
+    }
     const uint32_t nbig = sweep_big(sl);
     for (uint32_t k = blockIdx.x; k < nbig; k += gridDim.x) {
         uint32_t gid, v;
@@ -1907,10 +1930,31 @@ __device__ __forceinline__ bool tier1_hit_group(const GraphDev& g, bool mine, ui
     return group_bits(ballot(hit)) != 0;
 }
 
+template <bool ALONE>
 __global__ __launch_bounds__(256) void k_tier1_elem(const GraphDev* __restrict__ graphs, Space sp, SweepList sl,
                                                     int fresh, uint64_t* totals) {
     __shared__ uint32_t presence[BLOCK / WAVE][PRESENCE_WORDS];
     uint64_t rows = 0, slots = 0;
+    uint32_t cnt = 0, cur_gid = 0xFFFFFFFFu;
+    const auto count_for = [&](uint32_t gid) {   // conflicts counted from here on are graph gid's
+        if (gid == cur_gid) return;
+        if (cnt && lane() == 0) add32(&graphs[cur_gid].ctr[C_CONFLICTS], cnt);
+        cnt = 0;
+        cur_gid = gid;
+    };
+    if (ALONE) {
+        for_each_row(graphs, sp, [&](const GraphDev& g, uint32_t gid, uint32_t v) {
+            count_for(gid);
+            rows++;
+            slots += gp(g.fill)[v];
+            cnt += tier1_vertex(g, v, presence[threadIdx.x / WAVE], fresh);
+        });
+        if (cnt && lane() == 0) add32(&graphs[cur_gid].ctr[C_CONFLICTS], cnt);
+        if (lane() != 0) rows = slots = 0;
+        block_add64(totals, T_SWEEP_ROWS + 2, rows);
+        block_add64(totals, T_SWEEP_SLOTS + 2, slots);
+        return;
+    }
     const uint32_t nbig = sweep_big(sl);
     for (uint32_t k = blockIdx.x; k < nbig; k += gridDim.x) {
         uint32_t gid, v;
@@ -1924,14 +1968,9 @@ __global__ __launch_bounds__(256) void k_tier1_elem(const GraphDev* __restrict__
             slots += f;
         }
     }
-    uint32_t cnt = 0, cur_gid = 0xFFFFFFFFu;
     uint32_t row_n = 0, slot_n = 0;   // of the lane's rows (one lane of the row counts)
     for_rows(graphs, sp, sl, [&](const GraphDev& g, uint32_t gid, bool mine, uint32_t v) {
-        if (gid != cur_gid) {
-            if (cnt && lane() == 0) add32(&graphs[cur_gid].ctr[C_CONFLICTS], cnt);
-            cnt = 0;
-            cur_gid = gid;
-        }
+        count_for(gid);
         const uint32_t f = mine ? ld(&g.fill[v]) : 0u, s = mine ? gp(g.row_ptr)[v] : 0u;
         const uint32_t own = mine ? color_of(ld(&g.word[v])) : 0u, deg = mine ? gp(g.deg0)[v] : 0u;
         const bool one = mine && sublane() == 0;
@@ -2708,9 +2747,16 @@ hipError_t launch_build_list(const LaunchCtx& L, uint32_t kind, uint32_t* list, 
                                               L.active, L.gate);
     return hipGetLastError();
 }
+// Whether a sweep visits every row on a grid with a wavefront for each: the
+// kernel then takes them so, with the registers that takes (Tier-1: 64, with the
+// shared rows' and long rows' code 104, which leaves 4 wavefronts a SIMD, not 8).
+// Compaction and Tier-1 of 50,000 rows of 100 slots, us, so / with the shared
+// rows' code: 26 / 33 and 44 / 75.
+static inline bool alone_rows(const LaunchCtx& L) { return !L.list && L.V <= 4ull * sweep_grid(L); }
 hipError_t launch_compact(const LaunchCtx& L, bool drain_prep) {
-    k_compact<<<sweep_grid(L), 256, 0, L.stream>>>(L.graphs, space(L), sweep_list(L), L.totals,
-                                                   drain_prep ? L.ng : 0u, L.active);
+    auto* const kernel = alone_rows(L) ? &k_compact<true> : &k_compact<false>;
+    kernel<<<sweep_grid(L), 256, 0, L.stream>>>(L.graphs, space(L), sweep_list(L), L.totals, drain_prep ? L.ng : 0u,
+                                                L.active);
     return hipGetLastError();
 }
 hipError_t launch_drain(const LaunchCtx& L, bool serial, uint32_t max_count, bool prepped) {
@@ -2735,8 +2781,8 @@ hipError_t launch_tier1(const LaunchCtx& L, bool serial, int fresh) {
         const uint32_t grid = L.ng < 1024 ? L.ng : 1024;
         k_tier1_serial<<<grid, SERIAL_WAVES * WAVE, 0, L.stream>>>(L.graphs, L.ng, L.active, fresh, L.totals);
     } else {
-        k_tier1_elem<<<sweep_grid(L), 256, 0, L.stream>>>(L.graphs, space(L), sweep_list(L), fresh,
-                                                          L.totals);
+        auto* const kernel = alone_rows(L) ? &k_tier1_elem<true> : &k_tier1_elem<false>;
+        kernel<<<sweep_grid(L), 256, 0, L.stream>>>(L.graphs, space(L), sweep_list(L), fresh, L.totals);
     }
     return hipGetLastError();
 }

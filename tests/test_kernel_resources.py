@@ -1,4 +1,4 @@
-"""What the compiler gives the per-update kernels (CPU only: the device code is cross-compiled).
+"""What the compiler gives the hot kernels (CPU only: the device code is cross-compiled).
 
 A register that does not fit goes to scratch memory, a round trip for each use
 in a kernel that is one chain of round trips, and its time follows.
@@ -35,3 +35,11 @@ def test_per_update_kernels_use_no_scratch(kernel, resources):
     for name, r in mine.items():
         assert r["private_segment_fixed_size"] == 0 and r["vgpr_spill_count"] == 0, (name, r)
         assert r["vgpr_count"] <= 168, (name, r)   # three wavefronts a SIMD
+
+
+def test_full_sweeps_fill_the_chip(resources):
+    """Sweeps with a wavefront for every row: 8 wavefronts a SIMD, whatever the other variants take."""
+    mine = {n: r for n, r in resources.items() if re.search(r"k_(compact|tier1_elem)ILb1E", n)}
+    assert len(mine) == 2
+    for name, r in mine.items():
+        assert r["private_segment_fixed_size"] == 0 and r["vgpr_count"] <= 64, (name, r)
