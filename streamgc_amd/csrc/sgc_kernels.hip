@@ -2633,7 +2633,7 @@ constexpr uint32_t QUADS_OVER = 8192;
 // 325 / 197, of growth there 208 / 148; at one to 32, 16,384 of growth on a
 // 2^19-vertex one 142 / 152.
 constexpr uint32_t LONG_PER = 64;
-hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg,
+hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg,
                         uint64_t vertices) {
     if (count == 0) return hipSuccess;
     const bool group = eg && eg->keys && count > 1;
@@ -2651,19 +2651,28 @@ hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int
     else
         k_apply_elem<<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, count, multi, G.next, G.nheads, G.pack,
                                                   L.totals, L.dyn);
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    if (group && e == hipSuccess) eg->linked = false;
+    return e;
 }
 hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg) {
     k_group_clear<<<grid_for_waves(eg.size, 4 * WAVE, 1024), 256, 0, s>>>(eg.keys, eg.head, eg.size, eg.nheads);
     return hipGetLastError();
 }
-hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg) {
+// The table is full from the link to the apply launch of the same batch: if one
+// of the three did not start, the next batch clears it first (its entries and
+// counts would otherwise be taken for that batch's own).
+hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg) {
     if (count <= 1 || !eg || !eg->keys) return hipSuccess;
     if ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->pack) return hipErrorInvalidValue;
+    hipError_t e = eg->linked ? launch_group_clear(L.stream, *eg) : hipSuccess;
+    if (e != hipSuccess) return e;
+    eg->linked = true;
     const uint32_t mask = eg->size - 1;
     uint32_t mg = grid_for_waves(count, 4 * WAVE, 1024);
     k_group_link<<<mg, 256, 0, L.stream>>>(L.graphs, L.gbase, (const uint4*)upd, count, multi, eg->keys, eg->head,
                                            eg->next, mask, eg->heads, eg->next_cap, eg->nheads, L.dyn);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
     k_group_pack<<<mg, 256, 0, L.stream>>>((const uint4*)upd, eg->keys, eg->head, eg->next, eg->heads, eg->next_cap,
                                            eg->nheads, eg->pack, L.dyn);
     return hipGetLastError();

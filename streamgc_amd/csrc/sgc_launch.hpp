@@ -52,15 +52,16 @@ struct EdgeGroups {
     uint4* pack = nullptr;        // next_cap x 4 records: each listed edge's updates in stream order
     uint32_t size = 0;
     uint32_t next_cap = 0;
+    bool linked = false;          // a batch is in the table and its apply launch has not been issued
 };
 
 constexpr uint32_t GROUP_WORDS = 4;
-// Empties a new table (every batch leaves it empty).
+// Empties the table: a new one, or one that a failed launch left full (every other batch leaves it empty).
 hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg);
 // Per-edge grouping of a parallel batch (before launch_apply with the same eg).
-hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg);
+hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg);
 // vertices: of the graphs that the batch updates.
-hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, const EdgeGroups* eg,
+hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg,
                         uint64_t vertices);
 hipError_t launch_apply_seg(const LaunchCtx& L, const void* upd, const uint32_t* seg, uint32_t nseg,
                             const uint32_t* perm, int multi);
