@@ -272,7 +272,6 @@ struct sgc_pool {
     size_t t2_items_cap = 0;
     uint32_t* d_list = nullptr;           // sweep worklists (virtual vertex ids): the current sweep's, a later one's
     uint32_t* d_list_count = nullptr;     // their lengths
-    uint32_t ahead = NO_KIND;             // the later sweep whose worklist is built already
     uint32_t list_cap = 0;
     uint32_t ng = 0, V = 0;               // slots in use, vertices
     uint32_t act_n = 0, act_V = 0;        // active graphs and their vertices
@@ -469,19 +468,20 @@ struct sgc_pool {
     // `later`: the same set's sweep of that kind comes next and its worklist is
     // built in the same launches (nothing in between may mark a vertex for it
     // that is not sticky: compaction marks none, the drain only endpoints of
-    // overflowed edges).
-    hipError_t sweep(LaunchCtx& L, uint32_t kind, uint32_t later = NO_KIND) {
+    // overflowed edges).  `ahead` is the caller's note of that kind: the sweep
+    // that finds its own there takes the second list; it ends with the epoch.
+    hipError_t sweep(LaunchCtx& L, uint32_t kind, uint32_t* ahead = nullptr, uint32_t later = NO_KIND) {
         if (!tracking()) return hipSuccess;
         L.list = d_list;
         L.list_count = d_list_count;
         L.list_cap = list_cap;
-        if (kind == ahead) {
+        const bool built = ahead && *ahead == kind;
+        if (ahead) *ahead = built ? (uint32_t)NO_KIND : later;
+        if (built) {
             L.list += second_list();
             L.list_count += 2;
-            ahead = NO_KIND;
             return hipSuccess;
         }
-        ahead = later;
         return timed("build_list", [&] {
             return launch_build_list(L, kind, d_list, list_cap, d_list_count, later, second_list());
         });
@@ -542,12 +542,13 @@ struct sgc_pool {
     // ------------------------------------------------------------ hot path
     int apply(const sgc_edge_update* upd, uint32_t count, bool on_device, std::vector<uint64_t>& per_graph);
     int epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<sgc_epoch_stats>* out);
-    hipError_t rebuild(LaunchCtx L) {
-        hipError_t e = sweep(L, M_BITS);
+    int epoch_steps(const std::vector<uint32_t>& gids, bool finish, std::vector<sgc_epoch_stats>* out);
+    hipError_t rebuild(LaunchCtx L, uint32_t* ahead = nullptr) {
+        hipError_t e = sweep(L, M_BITS, ahead);
         if (e == hipSuccess) e = timed("rebuild", [&] { return launch_rebuild(L, exact_hist()); });
         return e;
     }
-    int tier1(const std::vector<uint32_t>& gids, uint32_t start_it = 0);
+    int tier1(const std::vector<uint32_t>& gids, uint32_t start_it = 0, uint32_t* ahead = nullptr);
     int tier2(const std::vector<uint32_t>& gids);
     int host_tier2(const std::vector<uint32_t>& list, std::vector<uint32_t>& ran);
     // Scratch of the device Tier-2's reverse-only neighbour list (12 bytes an entry).
@@ -824,7 +825,7 @@ void sgc_pool::drain_stats(const std::vector<uint32_t>& gids) {
 // iterating; each graph stops on its own (converged, plateau, iteration cap).
 // start_it > 0 continues a loop whose state (iterating, prev, plateau,
 // statistics) the caller has set: the sweeps a captured round ran.
-int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it) {
+int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it, uint32_t* ahead) {
     uint32_t max_iters = 0;
     for (uint32_t g : gids) {
         if (start_it == 0) {
@@ -850,7 +851,7 @@ int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it) {
             if (gs[g].iterating && fresh_level(g) < 2) reb.push_back(g);
         if (!reb.empty()) {
             e = set_active(reb);
-            if (e == hipSuccess) e = rebuild(ctx(true));
+            if (e == hipSuccess) e = rebuild(ctx(true), ahead);
         }
         if (e == hipSuccess) e = set_active_iterating(gids);
         LaunchCtx L = ctx(true);
@@ -874,7 +875,7 @@ int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it) {
                 e = set_active(part[serial][lvl]);
                 LaunchCtx L1 = ctx(true);
                 if (!serial) {
-                    if (e == hipSuccess) e = sweep(L1, M_CHECK);
+                    if (e == hipSuccess) e = sweep(L1, M_CHECK, ahead);
                     if (e == hipSuccess) e = timed("tier1", [&] { return launch_tier1(L1, false, lvl); });
                 } else if (e == hipSuccess) {
                     e = timed("tier1_serial", [&] { return launch_tier1(L1, true, lvl); });
@@ -1134,6 +1135,14 @@ int sgc_pool::max_colors(const std::vector<uint32_t>& gids) {
 // run_conflict_repair + cpu_serial_repair (A/src/streamgc.cu:1243-1423) and a
 // publish.  Statistics (out != null) cost a few extra synchronisations.
 int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<sgc_epoch_stats>* out) {
+    const int r = epoch_steps(gids, finish, out);
+    // A worklist's build clears the marks it lists, the one built ahead too: what a
+    // failed step left unswept is looked at again.
+    if (r && tracking())
+        for (uint32_t g : gids) (void)mark_all(g);
+    return r;
+}
+int sgc_pool::epoch_steps(const std::vector<uint32_t>& gids, bool finish, std::vector<sgc_epoch_stats>* out) {
     if (gids.empty()) return SGC_OK;
     for (uint32_t g : gids) {
         gs[g].st = sgc_epoch_stats();
@@ -1151,8 +1160,8 @@ int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<
         L = ctx(true);
     }
     LaunchCtx Lc = L;
-    ahead = NO_KIND;
-    if (e == hipSuccess) e = sweep(Lc, M_ROW, next_sweep(gids, repair));
+    uint32_t ahead = NO_KIND;   // the later sweep whose worklist is built already
+    if (e == hipSuccess) e = sweep(Lc, M_ROW, &ahead, next_sweep(gids, repair));
     if (e == hipSuccess) e = timed("compact", [&] { return launch_compact(Lc, true); });
     uint32_t ovf_cap = 0;
     for (uint32_t g : gids) ovf_cap = std::max(ovf_cap, gs[g].cfg.overflow_capacity);
@@ -1166,10 +1175,10 @@ int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<
         if ((r = read_drain(gids))) return r;
     if (repair) {
         if (finish && rebuild_each_sweep()) {
-            e = rebuild(L);
+            e = rebuild(L, &ahead);
             if (e != hipSuccess) return hip_fail(e, "rebuild");
         }
-        if ((r = tier1(gids))) return r;
+        if ((r = tier1(gids, 0, &ahead))) return r;
         if (out && swept) drain_stats(gids);
         if ((r = tier2(gids))) return r;
         if (!deterministic()) {   // bitmaps and histograms exact again for the next updates
@@ -1181,7 +1190,7 @@ int sgc_pool::epoch(const std::vector<uint32_t>& gids, bool finish, std::vector<
         if ((r = publish(gids))) return r;
         for (uint32_t g : gids) gs[g].settled = true;
     } else {
-        e = rebuild(L);
+        e = rebuild(L, &ahead);
         if (e != hipSuccess) return hip_fail(e, "rebuild");
     }
     if (out) {

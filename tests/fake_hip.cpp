@@ -61,7 +61,10 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, 
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind kind) { return hipMemcpyAsync(d, s, n, kind, nullptr); }
 hipError_t hipMemset(void* p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
-hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return hipMemset(p, v, n); }
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
+    launched.push_back("set");
+    return hipMemset(p, v, n);
+}
 
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }

@@ -15,6 +15,7 @@ from streamgc_amd import build
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 DRIVER = r"""
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include "fake_hip.hpp"
@@ -82,8 +83,51 @@ static void edge_table() {
     sgc_destroy(e);
 }
 
+static uint32_t* control = nullptr;   // the control block of a batched run, on the "device"
+
+// A captured round that stops for the host, its graph still iterating.
+static void watch(void* dst, const void*, size_t bytes, int kind) {
+    if (kind == (int)hipMemcpyHostToDevice && bytes == sgc::RC_WORDS * 4) control = (uint32_t*)dst;
+    if (kind == (int)hipMemcpyDeviceToHost && bytes == sizeof(sgc::RoundState))
+        *(sgc::RoundState*)dst = sgc::RoundState{1, 1000, 0, 2, 1000, 0};
+}
+static void stop() {
+    control[sgc::RC_ROUND] = 0;
+    control[sgc::RC_STOP] = 1;
+    control[sgc::RC_STOP_ROUND] = 0;
+}
+
+// The worklist an epoch builds ahead, for the sweep after its drain, is that epoch's alone.
+static void list_ahead() {
+    sgc_engine* e = path_engine();
+    sgc_batch_config c;
+    sgc_default_batch_config(&c);
+    uint32_t rounds = 0;
+    for (bool failed : {false, true}) {
+        CHECK(sgc_batch_prepare(e, recs.data(), recs.size(), &c, &rounds) == SGC_OK && rounds == 1);
+        sgc_epoch_stats st;
+        fake::launched.clear();
+        if (failed) fake::fail_next = "k_drain";
+        CHECK((sgc_epoch(e, &st) != SGC_OK) == failed && fake::fail_next.empty());
+        CHECK((at("k_rebuild") < 0) == failed);
+        CHECK((at("set") > at("k_list_tiles")) == failed);   // the listed vertices' marks are set again
+        fake::on_copy = watch;
+        fake::on_graph_launch = stop;
+        fake::launched.clear();
+        sgc_batch_stats bs;
+        CHECK(sgc_batch_run(e, &bs) == SGC_OK && bs.host_rounds == 1);
+        // the host's first sweep: the marked vertices are listed anew
+        const int graph = at("graph"), sweep = std::min((unsigned)at("k_rebuild", graph), (unsigned)at("k_tier1", graph));
+        CHECK(graph >= 0 && sweep > graph && at("k_list_tiles", graph) > graph && at("k_list_tiles", graph) < sweep);
+        fake::on_copy = nullptr;
+        fake::on_graph_launch = nullptr;
+    }
+    sgc_destroy(e);
+}
+
 int main() {
     edge_table();
+    list_ahead();
     std::printf("%s\n", fails ? "FAILED" : "ok");
     return fails ? 1 : 0;
 }
