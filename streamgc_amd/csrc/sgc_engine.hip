@@ -102,6 +102,7 @@ struct GraphState {
     sgc_config cfg{};
     uint32_t n = 0, nhd = 0;
     uint64_t S = 0;
+    uint64_t edges = 0, long_entries = 0;   // as loaded (see BatchGraphs)
     uint64_t bytes = 0;
     uint32_t *word = nullptr, *deg0 = nullptr, *row_ptr = nullptr, *col = nullptr, *hd_map = nullptr, *fill = nullptr;
     uint32_t *hubs = nullptr, *hist = nullptr, *ovf = nullptr;
@@ -202,7 +203,7 @@ struct BatchRun {
     sgc_batch_config cfg{};
     uint32_t rounds = 0, ng = 0, max_count = 0, sweeps = 0, ovf_cap = 0, t2_passes = 0;
     uint32_t sweeps_max = 0;                   // most Tier-1 sweeps a capture may hold
-    uint64_t max_vertices = 0;                 // of the graphs of the round with max_count records
+    BatchGraphs max_on;                        // the graphs of the round with max_count records
     uint64_t updates = 0;
     bool multi = false, any_history = false, all_settled = true;
     bool lean = false;                         // captures leave the Tier-2 check and repair out
@@ -486,10 +487,10 @@ struct sgc_pool {
             return launch_build_list(L, kind, d_list, list_cap, d_list_count, later, second_list());
         });
     }
-    uint64_t vertices(const std::vector<uint32_t>& gids) const {
-        uint64_t sum = 0;
-        for (uint32_t g : gids) sum += gs[g].n;
-        return sum;
+    BatchGraphs on(const std::vector<uint32_t>& gids) const {
+        BatchGraphs b;
+        for (uint32_t g : gids) b.vertices += gs[g].n, b.edges += gs[g].edges, b.long_entries += gs[g].long_entries;
+        return b;
     }
     size_t second_list() const { return list_words(list_cap, max_graphs); }
     // The sweep that follows an epoch's compaction and drain over the same
@@ -618,6 +619,11 @@ int sgc_pool::add_graph(const sgc_config* cfg, uint32_t n, const uint32_t* row_p
     G.cfg = *cfg;
     G.n = n;
     G.S = S;
+    G.edges = row_ptr[n] / 2;
+    for (uint32_t v = 0; v < n; v++) {
+        const uint32_t d = row_ptr[v + 1] - row_ptr[v];
+        if (d > HEAVY_FILL) G.long_entries += d;
+    }
     G.nhd = nhd;
     G.bytes = bytes;
     hipStream_t s = stream;
@@ -789,10 +795,11 @@ int sgc_pool::apply(const sgc_edge_update* upd, uint32_t count, bool on_device, 
         if (e == hipSuccess)
             e = timed("apply", [&] { return launch_apply_seg(L, src, seg.d, nseg, multi ? perm.d : nullptr, multi); });
     } else {
-        uint64_t verts = 0;
-        for (uint32_t g = 0; g < ng; g++) verts += per_graph[g] ? gs[g].n : 0u;
+        std::vector<uint32_t> gids;
+        for (uint32_t g = 0; g < ng; g++)
+            if (per_graph[g]) gids.push_back(g);
         e = timed("group", [&] { return launch_group(L, src, count, multi, &eg); });
-        if (e == hipSuccess) e = timed("apply", [&] { return launch_apply(L, src, count, multi, &eg, verts); });
+        if (e == hipSuccess) e = timed("apply", [&] { return launch_apply(L, src, count, multi, &eg, on(gids)); });
     }
     if (e != hipSuccess) return hip_fail(e, "apply launch");
     if (!on_device) {
@@ -1311,7 +1318,7 @@ int sgc_pool::batch_plan(const sgc_edge_update* upd, uint64_t count, const sgc_b
         B->tab.push_back((uint32_t)ordered.size() - off);
         if ((uint32_t)ordered.size() - off > B->max_count) {
             B->max_count = (uint32_t)ordered.size() - off;
-            B->max_vertices = vertices(in);
+            B->max_on = on(in);
         }
         B->gids.push_back(in);
         B->rounds++;
@@ -1453,7 +1460,7 @@ int sgc_pool::batch_capture(const sgc_tuning& t, hipGraphExec_t* out) {
         } else {
             e = launch_group(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg);
             if (e == hipSuccess)
-                e = launch_apply(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg, B.max_vertices);
+                e = launch_apply(La, B.d_stream, B.max_count, B.multi ? 1 : 0, &eg, B.max_on);
         }
     }
     LaunchCtx Lr = base;
@@ -1637,7 +1644,7 @@ int sgc_pool::batch_run_host(BatchRun& B) {
             e = timed("group", [&] { return launch_group(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg); });
             if (e == hipSuccess)
                 e = timed("apply", [&] {
-                    return launch_apply(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg, vertices(B.gids[r]));
+                    return launch_apply(L, B.d_stream + off, cnt, B.multi ? 1 : 0, &eg, on(B.gids[r]));
                 });
         }
         if (e != hipSuccess) return hip_fail(e, "batch apply");

@@ -356,7 +356,6 @@ __device__ __forceinline__ uint32_t key_hash(uint64_t k, uint32_t mask) {
 // 262K updates of 64 graphs of 2^10..2^15 vertices take 291 us with light
 // edges up to 64 slots, 257 up to 256 and 213 up to 1,024; a 131,072-vertex
 // mesh and the 4M-vertex power-law graph take the same with all three.
-constexpr uint32_t HEAVY_FILL = 1024;
 
 // The table is empty between batches: k_group_pack frees the slots it reads,
 // and k_apply_elem, which reads the counts that k_group_pack copied, clears the
@@ -2621,7 +2620,12 @@ static inline uint32_t grid_for_waves(uint64_t waves, uint32_t waves_per_block, 
 // 131,072-vertex mesh 107 / 58, an R-MAT graph of that size 285 / 269, of growth
 // 281 / 231, but 16,384 on a 32,768-vertex one 106 / 111; 196,608 of 48 graphs,
 // one to 2.4, 331 / 194).
-constexpr uint32_t QUADS_OVER = 8192;
+// Where more than three in ten edges are heavy, each of those takes a wavefront
+// either way, and the four-edge kernel pays only for more than QUADS_OVER_LONG:
+// 32,768 updates of an R-MAT graph of 262,144 vertices and 24 edges a vertex,
+// churn 225 / 219, growth 157 / 153, but the repairs that more updates in flight
+// cost make the growth's epochs 3% slower; 65,536 of growth there 295 / 230.
+constexpr uint32_t QUADS_OVER = 8192, QUADS_OVER_LONG = 32768;
 // A delete's long scans in trips of 1,024 slots for at most one update to
 // LONG_PER vertices.  They end a hub's deletes in half the time, and so before
 // other updates of the launch that touch the same vertices: on a skewed graph
@@ -2634,7 +2638,7 @@ constexpr uint32_t QUADS_OVER = 8192;
 // 2^19-vertex one 142 / 152.
 constexpr uint32_t LONG_PER = 64;
 hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg,
-                        uint64_t vertices) {
+                        const BatchGraphs& on) {
     if (count == 0) return hipSuccess;
     const bool group = eg && eg->keys && count > 1;
     if (group && ((uint64_t)eg->size < 2ull * count || eg->next_cap < count || !eg->heads || !eg->nheads || !eg->pack))
@@ -2642,10 +2646,11 @@ hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int
     const EdgeGroups G = group ? *eg : EdgeGroups();
     // one-wavefront blocks: a wavefront's slot is refilled as soon as it ends
     const uint32_t grid = grid_for_waves(count, 1, 4 * L.max_blocks);
-    if (group && count > QUADS_OVER && count <= vertices / LONG_PER)
+    if (group && count > QUADS_OVER && count <= on.vertices / LONG_PER)
         k_apply_quads<true><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
                                                          L.totals, L.dyn);
-    else if (group && count > QUADS_OVER && count <= vertices / 2)
+    else if (group && count > (10 * on.long_entries > 3 * on.edges ? QUADS_OVER_LONG : QUADS_OVER) &&
+             count <= on.vertices / 2)
         k_apply_quads<false><<<grid, WAVE, 0, L.stream>>>(L.graphs, (const uint4*)upd, multi, G.next, G.nheads, G.pack,
                                                           L.totals, L.dyn);
     else

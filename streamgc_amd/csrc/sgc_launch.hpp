@@ -60,9 +60,16 @@ constexpr uint32_t GROUP_WORDS = 4;
 hipError_t launch_group_clear(hipStream_t s, const EdgeGroups& eg);
 // Per-edge grouping of a parallel batch (before launch_apply with the same eg).
 hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg);
-// vertices: of the graphs that the batch updates.
+// Row slots past which an edge is listed as heavy (a wavefront of its own, first in the launch).
+constexpr uint32_t HEAVY_FILL = 1024;
+// The graphs that a batch updates: their vertices, undirected edges as loaded,
+// and the row entries of their vertices with more than HEAVY_FILL neighbours
+// (about as many as there are heavy edges).
+struct BatchGraphs {
+    uint64_t vertices = 0, edges = 0, long_entries = 0;
+};
 hipError_t launch_apply(const LaunchCtx& L, const void* upd, uint32_t count, int multi, EdgeGroups* eg,
-                        uint64_t vertices);
+                        const BatchGraphs& on);
 hipError_t launch_apply_seg(const LaunchCtx& L, const void* upd, const uint32_t* seg, uint32_t nseg,
                             const uint32_t* perm, int multi);
 hipError_t launch_zero_ctr(const LaunchCtx& L, uint32_t idx);

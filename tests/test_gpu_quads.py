@@ -97,14 +97,16 @@ def test_where_light_edges_go_by_four(pairs):
         assert np.array_equal(gpu.words() & 0xFFFF, orc.words() & 0xFFFF), (pairs, extra)
 
 
-def test_long_rows_in_sparse_launches():
-    """Long rows' searches in launches of few updates for the graph's size, among light edges that go by four."""
+@pytest.mark.parametrize("vertices,more", [(64, 0), (22, 80000), (4, 0)])
+def test_long_rows_among_light_edges(vertices, more):
+    """Long rows' searches in launches of light edges: by four with long trips (64 vertices to an update), by four
+    with short ones (a graph with few heavy edges), and one edge to a wavefront (most edges heavy)."""
     bed, pairs = 4000, 8200
     rng = np.random.default_rng(8)
     edges = [(bed + k, int(x)) for k, d in enumerate(test_gpu_apply.LONG) for x in rng.choice(bed, size=d, replace=False)]
     first = bed + len(test_gpu_apply.LONG)
-    edges += [(first + 2 * i, first + 2 * i + 1) for i in range(pairs)]
-    g = S.csr_from_edges(64 * (pairs + 100), edges)
+    edges += [(first + 2 * i, first + 2 * i + 1) for i in range(pairs + more)]
+    g = S.csr_from_edges(vertices * (pairs + 100), edges)
     gpu, orc, og = _pair(g, epoch_size=1 << 20, batch_size=1 << 20, slack_pct=3)
     u = first + 2 * np.arange(pairs, dtype=np.uint32)
     live = test_gpu_apply._live
