@@ -52,7 +52,7 @@ typedef struct sgc_edge_update {
 } sgc_edge_update;
 
 /* Engine flags. */
-#define SGC_DETERMINISTIC (1u << 0)      /* one wavefront, updates in stream order, repair in vertex order */
+#define SGC_DETERMINISTIC (1u << 0)      /* outcome of updates in stream order, repair in vertex order */
 #define SGC_REPAIR_EVERY_EPOCH (1u << 1) /* epoch = compact, drain, Tier-1, Tier-2, publish (proper snapshots) */
 #define SGC_EXACT_HISTOGRAM (1u << 2)    /* hub histograms recounted wherever bitmaps are rebuilt */
 #define SGC_FULL_SWEEPS (1u << 3)        /* maintenance sweeps visit every vertex (no dirty tracking); same results */
@@ -248,7 +248,7 @@ int sgc_kernel_times(sgc_engine* e, char* names, uint32_t name_stride, double* t
  * phase is one launch over all graphs taking part.  Records carry the graph
  * id in bytes 12..15 (sgc_edge_update.pad[3..6]).  Flags are pool-wide (the
  * sgc_config flags of sgc_pool_add are ignored).  Deterministic pools replay
- * each graph's updates in stream order on one wavefront per graph, so every
+ * each graph's updates to the outcome of stream order, slot for slot, so every
  * graph's result is the same alone and in the mix. */
 typedef struct sgc_pool sgc_pool;
 typedef struct sgc_pool_config {

@@ -1,7 +1,8 @@
 // sgc_device.hpp -- device-side layout and wave64 building blocks of the
 // StreamGC hot path for gfx950 (CDNA4).
 //
-// One 64-lane wavefront serves one edge update.  Row scans are lane-parallel
+// One 64-lane wavefront serves one edge update (the building blocks here; light
+// edges share a wavefront in sgc_kernels.hip).  Row scans are lane-parallel
 // (64 slots per load, coalesced); "first free or equal slot" and "first
 // match" are one __ballot each; the packed vertex word is claimed with a
 // 32-bit device-scope CAS; colour selection maps the 64-bit bitmap to a ffs

@@ -725,9 +725,9 @@ int sgc_pool::remove_graph(uint32_t gid) {
 
 // ============================================================== updates
 // One launch over a batch (local_update_kernel, A/src/streamgc.cu:847-854).
-// Parallel: one wavefront per update, same-edge updates grouped in stream
-// order.  Deterministic: one wavefront per graph, that graph's updates in
-// stream order.  per_graph receives the updates per graph.
+// Parallel: updates grouped by edge, an edge's in stream order, one edge or
+// four light ones to a wavefront.  Deterministic: each graph's updates to the
+// outcome of stream order.  per_graph receives the updates per graph.
 int sgc_pool::apply(const sgc_edge_update* upd, uint32_t count, bool on_device, std::vector<uint64_t>& per_graph) {
     per_graph.assign(ng, 0);
     if (count == 0) return SGC_OK;
@@ -866,8 +866,8 @@ int sgc_pool::tier1(const std::vector<uint32_t>& gids, uint32_t start_it, uint32
         // A graph sweeps in vertex order on one wavefront (Gauss-Seidel) when
         // deterministic, or when it is small and two parallel sweeps have left
         // a few conflicts (a racy sweep over a small conflict set can chase the
-        // same conflicts for many iterations); otherwise one wavefront per
-        // listed row.  Graphs of different selection levels take separate launches.
+        // same conflicts for many iterations); otherwise all listed rows at
+        // once.  Graphs of different selection levels take separate launches.
         std::vector<uint32_t> part[2][3];   // [serial][fresh level]
         for (uint32_t g : gids) {
             const GraphState& G = gs[g];

@@ -1,10 +1,12 @@
 // sgc_kernels.hip -- HIP kernels of the StreamGC hot path for gfx950.
 //
-// Work decomposition: updates are one wavefront each (grid-stride), or one
-// wavefront per segment replayed in order (deterministic mode).  Epoch sweeps
-// run one wavefront per vertex row over the vertex space of the graphs taking
-// part (their vertex counts laid end to end); rows are streamed 64
-// slots per load.  The deterministic repair sweep runs one wavefront per
+// Work decomposition: a parallel batch's updates are grouped by edge, an edge
+// to a wavefront or four light edges to one; deterministic batches replay each
+// graph's segment by a block of wavefronts (one wavefront where there are very
+// many segments).  Epoch sweeps run over the vertex rows of the graphs taking
+// part (their vertex counts laid end to end), one to four short rows to a
+// wavefront, a longer row to a wavefront, the longest to a block; rows are
+// streamed 64 slots per load.  The deterministic repair sweep runs one block per
 // graph in vertex order.
 #include <hip/hip_runtime.h>
 
@@ -46,17 +48,17 @@ __device__ __forceinline__ Space device_space(const uint32_t* dspace, uint32_t n
 }
 
 // ---------------------------------------------------------------- sweep sets
-// A maintenance sweep visits either every virtual vertex (list == null, one
-// wavefront per row) or the worklist launch_build_list left on the device.
+// A maintenance sweep visits either every virtual vertex (list == null) or the
+// worklist launch_build_list left on the device.
 // The worklist keeps rows of at most `long_row` filled slots at its front
-// (count[0] of them, one wavefront each) and longer rows at its back
+// (count[0] of them, for_rows) and longer rows at its back
 // (count[1], list[cap - 1 - k], one 256-thread block each), so a hub row
 // costs a few block-wide round trips instead of hundreds of wavefront ones.
 // Lengths are read on the device: the host never waits for them.
 constexpr uint32_t BLOCK = 256;
 
 struct SweepList {
-    const uint32_t* list;   // null: every vertex, wavefront per row
+    const uint32_t* list;   // null: every vertex
     const uint32_t* count;  // [small, big]
     uint32_t cap;
 };
@@ -72,8 +74,9 @@ __device__ __forceinline__ uint32_t big_item(const SweepList& sl, uint32_t k) { 
 // share of the rows.  A full sweep of 4.0M rows and 69M live
 // slots, one row a wavefront / four: compaction 1,180 / 324 us, rebuild 2,200 /
 // 1,137 us, Tier-1 3,513 / 1,071 us (what is left is the gather of 69M
-// neighbour words).  body(g, gid, mine, v) runs with g wave-uniform (rows of several graphs: one graph after another): mine says
-// whether the lane's row v takes part.
+// neighbour words).  body(g, gid, mine, v) runs with g wave-uniform (rows of
+// several graphs: one graph after another); mine says whether the lane's row v
+// takes part.
 constexpr uint32_t GROUP = 16, GROUPS = WAVE / GROUP;
 constexpr uint32_t GROUP_ROW = ROW_UNROLL * GROUP;   // slots 16 lanes load in one round trip
 __device__ __forceinline__ uint32_t sublane() { return lane() % GROUP; }
@@ -389,7 +392,7 @@ __device__ __forceinline__ uint32_t group_slot(uint64_t* __restrict__ keys, uint
 // Links every update of the batch into its edge's list, and lists each edge
 // once (the update that inserted the key adds its slot; an update whose key
 // found no slot is listed alone, position | GROUP_SINGLE): the per-update
-// kernel then runs one wavefront per edge.  Records that change nothing
+// kernels then take one edge after another.  Records that change nothing
 // (out-of-range vertex, other kinds) are not listed.  Each block appends its
 // entries with one atomic per list end; nheads = [heavy, light] counts, and
 // k_group_pack's copy of them.
@@ -572,7 +575,10 @@ __device__ __forceinline__ void apply_edge(const GraphDev* __restrict__ graphs, 
     grouped += applied ? applied - 1 : 0;
 }
 
-// One wavefront per edge of the batch.
+// One wavefront per edge of the batch.  Bound: the chain of an edge's dependent
+// gathers and atomics, 165 registers (3 wavefronts a SIMD).  4,099 updates of a
+// 131,072-vertex mesh 16 us, of a 65,536-vertex R-MAT graph 45 us (its hub rows'
+// scans).
 __global__ __launch_bounds__(64) void k_apply_elem(const GraphDev* __restrict__ graphs, const uint4* __restrict__ upd,
                                                    uint32_t count, int multi, const uint32_t* __restrict__ gnext,
                                                    uint32_t* __restrict__ nheads, const uint4* __restrict__ pack,
@@ -880,9 +886,12 @@ __device__ __forceinline__ void apply_quad(const GraphDev& g, bool act, const ui
 }
 
 // One wavefront per heavy edge of the batch, then one per four light ones (if
-// they are enough to fill the chip, some 3,000 wavefronts of this kernel).
-// Bound: the chain of dependent gathers and atomics of an edge, over the
-// wavefronts the registers allow.
+// they are enough to fill the chip, some 3,000 wavefronts of this kernel: 168
+// registers, no scratch).  Bound: the chain of dependent gathers and atomics of
+// four edges, over the wavefronts the registers allow.  One edge a wavefront /
+// this kernel: 32,768 updates of a 131,072-vertex mesh 57 / 39 us, of a
+// 262,139-vertex power-law graph 70 / 49, of a 4M-vertex one 125 / 78 (with LONG),
+// 196,608 of 48 graphs 331 / 194.
 constexpr uint32_t APPLY_SPREAD = 4096;
 template <bool LONG>
 __global__ __launch_bounds__(64, 3) void k_apply_quads(const GraphDev* __restrict__ graphs,
@@ -1240,10 +1249,8 @@ __global__ __launch_bounds__(256) void k_snapshot(const GraphDev* __restrict__ g
 
 // ---------------------------------------------------------------- compaction
 // A/src/kernels/epoch_maintenance.cu:20-61: stable left-pack of the live
-// slots, free slots after them.  One pass, writing only slots whose content
-// changes: a live value moves to w + (live lanes before it); a slot whose
-// value moved and that lies past the chunk's new write front is freed (a
-// later chunk may refill it, in program order).
+// slots, free slots after them.
+
 // A block barrier for data in LDS: outstanding global loads and stores go on
 // across it (__syncthreads waits for them).
 __device__ __forceinline__ void lds_barrier() {
@@ -1317,7 +1324,10 @@ __device__ __forceinline__ uint32_t compact_row_block(const GraphDev& g, uint32_
     return w - s;
 }
 
-// One row, one wavefront: ROW_UNROLL chunks loaded, then packed in order.
+// One row, one wavefront: ROW_UNROLL chunks loaded, then packed in order, in one
+// pass that writes only slots whose content changes: a live value moves to w +
+// (live lanes before it); a slot whose value moved and that lies past the chunk's
+// new write front is freed (a later chunk may refill it, in program order).
 __device__ __forceinline__ uint32_t compact_row_wave(const GraphDev& g, uint32_t v) {
     const uint64_t lt_mask = (1ull << lane()) - 1ull;
     const uint32_t s = gp(g.row_ptr)[v], e = s + gp(g.fill)[v];
@@ -1385,7 +1395,9 @@ __device__ __forceinline__ void drain_prep_graph(const GraphDev* __restrict__ gr
 }
 
 // (256, 8): with more than 64 registers only 7 of a CU's 8 blocks of the usual
-// grid run at once, and a full sweep waits for the eighth (327 -> 526 us).
+// grid run at once, and a full sweep waits for the eighth (327 -> 526 us).  The
+// long rows' windows pay for it: 2 vector registers (12 B of scratch a lane) and
+// 56 scalar ones are spilled around compact_row_block.
 // prep_ng > 0: block 0 also takes the drain's counter snapshot of the
 // active graphs (k_drain_prep), which the drain launched next reads;
 // compaction touches none of those counters.
@@ -2729,9 +2741,9 @@ hipError_t launch_snapshot(const LaunchCtx& L, const uint32_t* fl_round, const H
     k_snapshot<<<grid, 256, 0, L.stream>>>(L.graphs, space(L), L.active, fl_round, hist);
     return hipGetLastError();
 }
-// Sweep grids: one wavefront per row (blocks first take the long rows of a
-// worklist), grid-stride; a worklist sweep takes the grid of a full sweep
-// capped at sweep_blocks (its length is on the device).
+// Sweep grids: a wavefront per row up to a cap, grid-stride (blocks first take
+// the long rows of a worklist); a worklist sweep's cap is sweep_blocks (its
+// length is on the device).
 static inline uint32_t sweep_grid(const LaunchCtx& L) {
     return grid_for_waves(L.V, 4, L.list ? L.sweep_blocks : L.max_blocks);
 }
