@@ -1115,7 +1115,8 @@ __global__ __launch_bounds__(WAVES * WAVE) void k_apply_seg(const GraphDev* __re
                         i0 += run;
                         run = 0;
                     }
-                    for (uint32_t i = at; i < at + mine; i++) apply_rec(graphs, uniform_rec(w.recs[i]), multi, acc);
+                    for (uint32_t i = at; i < at + mine; i++)   // (long scans: the order is the stream's anyway)
+                        apply_rec<true>(graphs, uniform_rec(w.recs[i]), multi, acc);
                     __syncthreads();
                 }
                 i0 += stop;
@@ -2694,7 +2695,7 @@ hipError_t launch_group(const LaunchCtx& L, const void* upd, uint32_t count, int
                                            eg->nheads, eg->pack, L.dyn);
     return hipGetLastError();
 }
-// A CU holds 20 wavefronts of this kernel: one block of REPLAY_WAVES, or two of
+// A CU holds 16 wavefronts of this kernel: one block of REPLAY_WAVES, or two of
 // half as many.  Up to REPLAY_BLOCKS segments (one to a CU) take whole blocks, up
 // to twice as many half ones, above it one wavefront each: a segment that had to
 // wait for another's block would take twice as long, which a stream with nothing
