@@ -128,7 +128,7 @@ def kernel_bytes(name, launches, n, tot, live_frac):
     return 0
 
 
-ROCPROF_NAMES = {"apply": "k_apply_elem", "group": "k_group_link", "rebuild": "k_rebuild", "tier1": "k_tier1_elem",
+ROCPROF_NAMES = {"apply": "k_apply_quads", "group": "k_group_link", "rebuild": "k_rebuild", "tier1": "k_tier1_elem",
                  "tier1_serial": "k_tier1_serial",
                  "compact": "k_compact", "build_list": "k_list_tiles", "snapshot": "k_snapshot"}
 
