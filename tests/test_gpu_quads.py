@@ -126,3 +126,31 @@ def test_long_rows_among_light_edges(vertices, more):
         got, want = gpu.csr()[1], orc.csr()[1]
         assert np.array_equal(got, want), (k, np.nonzero(got != want)[0][:8])
     assert gpu.overflow_count() == orc.overflow_count()
+
+
+@pytest.mark.parametrize("order", [{"repair_every_epoch": True}, {}])
+def test_shared_vertices_keep_every_invariant(order):
+    """Churn and growth whose updates share vertices at random: the live edges are the oracle's, every bitmap
+    row's bits hold its neighbours' colours, and a repaired epoch is proper."""
+    g = S.gen_chung_lu(40000, 200000, 2.3, 300.0, seed=3, permute=True)
+    gpu, orc, og = _pair(g, epoch_size=12000, batch_size=12000, exact_histogram=True, histogram_threshold=40, **order)
+    init = S.generate_init_stream(g)
+    gpu.process_stream(init)
+    gpu.finish()
+    orc.submit(init["u"], init["v"], init["type"])
+    orc.finish()
+    for stream in (S.generate_bench_stream_edges(g, 24000, 50, 6), S.dense_growth_stream(g, 24000, seed=7)):
+        gpu.process_stream(stream)
+        orc.submit(stream["u"], stream["v"], stream["type"])
+        if not order:
+            gpu.finish()
+        assert gpu.overflow_count() == orc.overflow_count() == 0
+        assert gpu.validate()[:2] == (0, 0)
+        rp, col = gpu.csr()
+        row = np.repeat(np.arange(g.n), np.diff(rp.astype(np.int64)))
+        live = col != 0xFFFFFFFF
+        assert np.array_equal(_rows((rp, col)), _rows(orc.csr()))
+        colour = gpu.colors().astype(np.int64)[col[live]]
+        held = gpu.bitmaps()[row[live]]
+        few = (colour <= 64) & (g.degree[row[live]] <= 40)   # (histogram rows' bitmaps are never rebuilt)
+        assert np.all(held[few] >> (colour[few] - 1).astype(np.uint64) & np.uint64(1))
